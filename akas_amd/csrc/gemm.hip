@@ -6,6 +6,7 @@
 #include "device_info.h"
 #include "gemm_core.h"
 #include "gemm_dma.h"
+#include "gemm_pipe.h"
 #include "quant_group.h"
 
 namespace akas {
@@ -37,7 +38,8 @@ AKAS_DEV void grouped_tile(int id, int tiles_m, int tiles_n, int G, int& tm, int
 }
 
 // ---------------------------------------------------------------------------
-// LDS-tiled MFMA GEMM (prefill shapes and medium M)
+// LDS-tiled MFMA GEMM staged through registers, for operands that the DMA
+// kernels below do not take
 //
 // DEPTH k-blocks are in flight per workgroup in a register ring in front of
 // the two LDS stages: at k-block kb the ring holds kb+1 .. kb+DEPTH, so the
@@ -523,6 +525,75 @@ __global__ __launch_bounds__(dma::THREADS) void dense_dma_kernel(DenseArgs p) {
 }
 
 // ---------------------------------------------------------------------------
+// The pipelined engine (gemm_pipe.h) on a dense product: any M, N a multiple
+// of 16 (rows and columns past the ends are clamped on load and never
+// stored), up to kPipeMaxKb k-blocks per partition.  A wave's columns sit in
+// one 128-column scale block, whose scales it holds in registers (lane l
+// those of k-blocks l and 64 + l).
+// ---------------------------------------------------------------------------
+constexpr int kPipeMaxKb = 128;
+
+struct DensePipePlan {
+  const uint8_t* a_base;
+  const uint8_t* b_base;
+  const float* as;
+  uint32_t a_off[4], b_off[4], s_off;
+  AKAS_DEV const uint8_t* a(int i, int kb) const { return a_base + (int64_t)kb * kBlock + a_off[i]; }
+  AKAS_DEV const uint8_t* b(int i, int kb) const { return b_base + (int64_t)kb * kBlock + b_off[i]; }
+  AKAS_DEV const float* s(int kb) const { return as + kb + s_off; }
+};
+
+template <class E, int OUT, int SDT>
+__global__ __launch_bounds__(E::THREADS) void dense_pipe_kernel(DenseArgs p) {
+  const int tiles_m = (p.M + E::BM - 1) / E::BM, tiles_n = (p.N + E::BN - 1) / E::BN;
+  const int id = xcd_remap(blockIdx.x, tiles_m * tiles_n);
+  int tm, tn;
+  grouped_tile(id, tiles_m, tiles_n, 8, tm, tn);
+  const int m0 = tm * E::BM, n0 = tn * E::BN;
+  const int KB = p.K / kBlock, nkb = p.kb_per_part;
+  const int part = blockIdx.y, kb0 = part * nkb;
+
+  const E e(threadIdx.x);
+  float wreg[2];
+  {
+    const int64_t base = (int64_t)min((n0 + e.b_row0) / kBlock, (p.N - 1) / kBlock) * KB + kb0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) wreg[h] = load_scale_t<SDT>(p.ws, base + min(e.lane + 64 * h, nkb - 1));
+  }
+  DensePipePlan plan;
+  static_assert(E::PA <= 4 && E::PB <= 4, "offsets of the plan");
+  plan.a_base = p.a;
+  plan.b_base = p.w;
+  plan.as = p.as;
+#pragma unroll
+  for (int i = 0; i < E::PA; ++i) {
+    const int row = e.a_piece_row(i);
+    plan.a_off[i] = (uint32_t)min(m0 + row, p.M - 1) * (uint32_t)p.K + e.piece_chunk(row);
+  }
+#pragma unroll
+  for (int i = 0; i < E::PB; ++i) {
+    const int row = e.b_piece_row(i);
+    plan.b_off[i] = (uint32_t)min(n0 + row, p.N - 1) * (uint32_t)p.K + e.piece_chunk(row);
+  }
+  plan.s_off = (uint32_t)min(m0 + e.scale_row(), p.M - 1) * (uint32_t)KB;
+
+  typename E::Acc acc;
+  acc.clear();
+  e.template run<false>(plan, acc, kb0, nkb, [&](int kb) {
+    const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kb < 64 ? wreg[0] : wreg[1]), kb & 63));
+    return float2{w, w};
+  });
+  const int64_t obase = (int64_t)part * p.part_stride;
+  constexpr int kPer16 = OUT == AKAS_DTYPE_F32 ? 4 : 8;  // output elements per 16 bytes
+  const bool wide = p.ldo % kPer16 == 0 && p.part_stride % kPer16 == 0 &&
+                    reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
+  e.reduce(acc, [&](int row, int col, const v4f& lo, const v4f& hi) {
+    if (m0 + row < p.M && n0 + col < p.N)
+      pipe::store_out8<OUT>(p.out, obase + (int64_t)(m0 + row) * p.ldo + n0 + col, lo, hi, wide);
+  });
+}
+
+// ---------------------------------------------------------------------------
 // Small-M MFMA GEMM: one 16-column tile per workgroup, four waves striding
 // over the k-blocks with every operand fetched straight from global memory
 // (weights stream once from HBM, activations hit L2), then a fixed-order
@@ -624,7 +695,7 @@ __global__ __launch_bounds__(256) void dense_small_kernel(DenseArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// Wide small-M MFMA GEMM (M <= 64): one workgroup of NTW x KS waves covers
+// Wide small-M MFMA GEMM (M <= 32): one workgroup of NTW x KS waves covers
 // 16*NTW columns and the partition's whole k range.  The activation slab
 // (codes and scales of all its rows) is staged in LDS once per workgroup,
 // every wave issues all of its weight loads up front (k-blocks strided by
@@ -840,14 +911,79 @@ static void launch_tiled(const DenseArgs& a, int parts, hipStream_t s) {
       <<<dim3(tiles, parts), 64 * WMW * WNW, 0, s>>>(a);
 }
 
-// The DMA-fed 256x256 kernel takes over once its tiles cover the GPU at
-// least about once (fewer, larger tiles idle too many CUs) and the output
-// rows are 16-byte aligned for its vector stores.
-static bool dma_fits(const DenseArgs& a, int parts) {
+// What the DMA-fed 256x256 kernel accepts: whole 128-column blocks and output
+// rows aligned for its 16-byte stores.
+static bool dma_fits(const DenseArgs& a) {
   const int esz = a.out_dtype == AKAS_DTYPE_F32 ? 4 : 2;
-  const int64_t tiles = (int64_t)((a.M + dma::BM - 1) / dma::BM) * ((a.N + dma::BN - 1) / dma::BN);
-  return a.N % 128 == 0 && tiles * parts >= 240 && a.kb_per_part <= dma::MAX_KB && (a.ldo * esz) % 16 == 0 &&
+  return a.N % 128 == 0 && a.kb_per_part <= dma::MAX_KB && (a.ldo * esz) % 16 == 0 &&
          (a.part_stride * esz) % 16 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0;
+}
+
+// What the pipelined engine accepts: its DMA takes 16-byte aligned codes
+// (rows are multiples of 128 bytes, so aligned bases suffice).
+static bool pipe_fits(const DenseArgs& a) {
+  return a.kb_per_part <= kPipeMaxKb && reinterpret_cast<uintptr_t>(a.a) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(a.w) % 16 == 0;
+}
+
+// Tiles of the pipelined engine, by workgroups per CU: small tiles in many
+// k-block groups cover the CUs at few rows, 128x128 tiles move the fewest
+// bytes per product, and two of them per CU overlap each other's barriers.
+using Pipe64x64 = pipe::Engine<64, 64, 2, 2, 2, 4>;
+using Pipe64x128 = pipe::Engine<64, 128, 2, 2, 2, 3>;
+using Pipe128x128 = pipe::Engine<128, 128, 2, 2, 2, 2>;
+using Pipe128x128x2 = pipe::Engine<128, 128, 2, 2, 1, 2>;
+
+template <class E, int OUT, int SDT>
+static void launch_pipe(const DenseArgs& a, int parts, hipStream_t s) {
+  const int tiles = ((a.M + E::BM - 1) / E::BM) * ((a.N + E::BN - 1) / E::BN);
+  dense_pipe_kernel<E, OUT, SDT><<<dim3(tiles, parts), E::THREADS, 0, s>>>(a);
+}
+
+// Estimated time in us of a tiled launch: a launch constant, and per round of
+// workgroups a constant and a rate per k-block (with one, or with two,
+// workgroups on the busiest CU).  Fitted to launches of every kernel at 19
+// row counts from 33 to 8192 and eight (K, N) from 1024x1024 to 8192x2048
+// (root-mean-square error 5-7%); taking the least estimate came within 0.4%
+// on average, and 7% at worst, of the fastest kernel over them.  (The
+// 256x256 kernel's rounds after the first cost more than its first: with
+// every CU busy the card runs at a lower clock.)
+enum DenseTile { kTile64x64, kTile64x128, kTile128x128, kTile128x128x2, kTile256x256, kDenseTiles };
+struct DenseTileCost {
+  int bm, bn, per_cu;
+  float launch, round, kb1, kb2;
+};
+constexpr DenseTileCost kDenseTileCost[kDenseTiles] = {
+    {64, 64, 1, 1.5f, 2.6f, 0.256f, 0.f},     {64, 128, 1, 1.6f, 2.6f, 0.365f, 0.f},
+    {128, 128, 1, 0.5f, 3.4f, 0.577f, 0.f},   {128, 128, 2, 2.2f, 1.5f, 0.718f, 1.113f},
+    {256, 256, 1, -7.8f, 12.9f, 1.375f, 0.f},
+};
+
+static float dense_cost(const DenseTileCost& c, const DenseArgs& a, int parts) {
+  const int64_t cus = device_cus();
+  const int64_t tiles = (int64_t)((a.M + c.bm - 1) / c.bm) * ((a.N + c.bn - 1) / c.bn) * parts;
+  const int64_t full = tiles / (cus * c.per_cu), rest = tiles % (cus * c.per_cu);
+  float t = c.launch + (full + (rest > 0)) * c.round +
+            full * a.kb_per_part * (c.per_cu == 2 ? c.kb2 : c.kb1);
+  if (rest > 0) t += a.kb_per_part * (rest > cus ? c.kb2 : c.kb1);
+  return t;
+}
+
+// The tile with the least estimate, and the estimate.  The 256x256 kernel is
+// for prefill (above 256 rows), where it fits.
+static DenseTile dense_tile(const DenseArgs& a, int parts, float* cost = nullptr) {
+  int best = kTile64x64;
+  float least = dense_cost(kDenseTileCost[best], a, parts);
+  for (int i = best + 1; i < kDenseTiles; ++i) {
+    if (i == kTile256x256 && (a.M <= 256 || !dma_fits(a))) continue;
+    const float t = dense_cost(kDenseTileCost[i], a, parts);
+    if (t < least) {
+      least = t;
+      best = i;
+    }
+  }
+  if (cost) *cost = least;
+  return (DenseTile)best;
 }
 
 // The split kernel: 2048-deep partitions, N a multiple of its 48-column
@@ -872,8 +1008,26 @@ static bool split_fits(const DenseArgs& a) {
          reinterpret_cast<uintptr_t>(a.as) % 16 == 0;
 }
 
+// Rows of a split workgroup's tile by M (see launch_split_m).
+static int split_rows(int m) { return m <= 32 ? 16 : m <= 64 ? 32 : m <= 128 ? 64 : 128; }
+
+// The split kernel takes the decode batches it fits unless the pipelined
+// engine is estimated faster.  Up to 32 rows it is the faster one everywhere
+// (K=8192, N=6144, M=32: 22.3 us, 27.0 pipelined), up to 128 while at most
+// two of its workgroups come to a CU (fp8_linear, K=2048, N=8192: M=64
+// 9.4 us, 11 pipelined; M=128 11.0, 11.4).  Beyond, its time is 4.2 us and its
+// operand bytes per CU at 70 KB per us (measured from 300 to 900 KB per CU):
+// N=8192, M=256 15.9 us, 13.5 pipelined; K=8192, N=6144, M=100 31.5, 27.1.
 static bool split_applies(const DenseArgs& a, int parts) {
-  return a.M > 16 && a.M <= 256 && split_fits(a) && parts >= 1;
+  if (a.M <= 16 || a.M > 256 || !split_fits(a) || parts < 1) return false;
+  const int nt = split_nt(a), rows = split_rows(a.M), row_tiles = (a.M + rows - 1) / rows;
+  const int64_t blocks = (int64_t)(a.N / (16 * nt)) * parts;
+  if (a.M <= 32 || (a.M <= 128 && blocks * row_tiles <= 2 * (int64_t)device_cus()) || !pipe_fits(a))
+    return true;
+  const float bytes = (float)blocks * (row_tiles * 16 * nt + a.M) * (a.kb_per_part * kBlock);
+  float cost;
+  dense_tile(a, parts, &cost);
+  return 4.2f + bytes / 1024.f / device_cus() / 70.f <= 1.1f * cost;
 }
 
 template <int MT, int PF, int AFIRST, int AF, int OUT, int SDT, int MH = 1, int NT = kSplitNt>
@@ -977,40 +1131,46 @@ static bool launch_wide_m16(const DenseArgs& a, int parts, hipStream_t s) {
   }
 }
 
+// Products of at most 64 rows and few k-blocks, while the direct small
+// kernel's 16-column workgroups fit the CUs once: it has no stages to fill
+// (K=1024, N=2048, M=32: 4.6 us against 5.3 on the pipelined engine; K=512,
+// M=40: 4.4, 4.4; K=1024, M=40: 5.4, 5.4; K=3072, M=32: 9.6, 9.3).
+static bool shallow_rows(const DenseArgs& a) {
+  return a.M <= 64 && a.kb_per_part <= (a.M <= 32 ? 12 : 4) && a.N <= 16 * device_cus();
+}
+
 // Kernel choice by shape, in order:
-//   16 < M <= 256 with 2048-deep partitions   the split kernel
-//   M <= 64                                   the wide kernel (activations
-//                                             staged once per workgroup in LDS),
-//                                             else the direct small kernel
-//   M > 256 whose 256x256 tiles fill the GPU  the DMA-fed prefill kernel
-//   otherwise                                 64x64 tiles up to 256 rows, then
-//                                             256x128 tiles when they fill the
-//                                             GPU, else 128x128
-// Tiled kernels need N to be a multiple of BN (affine B rows); shapes that
-// fit none of these fall back to 64-row slices of the direct small kernel.
+//   M <= 16                                   the wide kernel (activations
+//                                             staged once per workgroup in LDS)
+//   16 < M <= 256 with 2048-deep partitions   the split kernel, where estimated
+//                                             faster than the engine below
+//   16 < M <= 64, few k-blocks                the direct small kernel (shallow_rows)
+//   16 < M <= 32, 9 to 16 k-blocks, columns   the wide kernel (K=1536, N=6144,
+//     past one 16-column tile per CU          M=24: 6.6 us, 7.0 pipelined)
+//   otherwise                                 the pipelined engine or the 256x256
+//                                             DMA kernel, the tile estimated fastest
+// Codes off 16-byte alignment and partitions past kPipeMaxKb k-blocks take
+// the register-staged kernels: 128x128 tiles where N is a multiple of 128,
+// else (and up to 64 rows) the direct small kernel in 64-row slices.
 template <int OUT, int SDT>
 static void launch_dense_t(const DenseArgs& a, int parts, hipStream_t s) {
-  bool done = false;
+  if (a.M <= 16 && launch_wide_m16<OUT, SDT>(a, parts, s)) return;
   if (split_applies(a, parts)) {
     launch_split_m<0, OUT, SDT>(a, parts, s);
     return;
   }
-  if (a.M <= 16)
-    done = launch_wide_m16<OUT, SDT>(a, parts, s);
-  else if (a.M <= 32)
-    done = launch_wide<2, 2, 8, OUT, SDT>(a, parts, s);
-  else if (a.M <= 64)
-    done = launch_wide<4, 2, 8, OUT, SDT>(a, parts, s);
-  if (done) return;
-  if (a.M <= 64) {
-    launch_small<OUT, SDT>(a, parts, s);
-  } else if (a.M > 256 && dma_fits(a, parts)) {
-    launch_dma<OUT, SDT>(a, parts, s);
-  } else if (a.M <= 256 && a.N % 64 == 0) {
-    launch_tiled<64, 64, 2, 2, 2, OUT, SDT>(a, parts, s);
-  } else if (a.N % 128 == 0 && (int64_t)((a.M + 255) / 256) * (a.N / 128) >= 512) {
-    launch_tiled<256, 128, 4, 2, 1, OUT, SDT>(a, parts, s);
-  } else if (a.N % 128 == 0) {
+  if (a.M <= 32 && a.kb_per_part > 8 && a.kb_per_part <= 16 && a.N > 16 * device_cus() &&
+      launch_wide<2, 2, 8, OUT, SDT>(a, parts, s))
+    return;
+  if (a.M > 16 && pipe_fits(a) && !shallow_rows(a)) {
+    switch (dense_tile(a, parts)) {
+      case kTile64x64: launch_pipe<Pipe64x64, OUT, SDT>(a, parts, s); break;
+      case kTile64x128: launch_pipe<Pipe64x128, OUT, SDT>(a, parts, s); break;
+      case kTile128x128: launch_pipe<Pipe128x128, OUT, SDT>(a, parts, s); break;
+      case kTile128x128x2: launch_pipe<Pipe128x128x2, OUT, SDT>(a, parts, s); break;
+      default: launch_dma<OUT, SDT>(a, parts, s);
+    }
+  } else if (a.M > 64 && a.N % 128 == 0) {
     launch_tiled<128, 128, 2, 2, 1, OUT, SDT>(a, parts, s);
   } else {
     const int esz = OUT == AKAS_DTYPE_F32 ? 4 : 2;
@@ -1167,13 +1327,20 @@ static int run_fp8_linear(const void* x, int x_dtype, const uint8_t* w, const vo
                                               align256((size_t)r * (k / kBlock) * sizeof(float)));
     DenseArgs p{codes, scales, w, w_scales, partial, (int64_t)parts * o, o, (int)r, (int)o,
                 (int)k, (int)(k / kBlock / parts), scale_dtype, AKAS_DTYPE_F32, nullptr, 0};
-    if (split_applies(p, parts)) {
-      const int st = launch_quantize(x, x_dtype, codes, scales, r, k, true, s);
+    // the kernel that akas_projection_partial takes for these partitions, so
+    // that the result is that of the partial and merge pair bit for bit
+    if (split_fits(p)) {
+      const bool frag = split_applies(p, parts);
+      int st = launch_quantize(x, x_dtype, codes, scales, r, k, frag, s);
       if (st != AKAS_OK) return st;
-      if (scale_dtype == AKAS_DTYPE_F32)
+      if (!frag) {
+        st = launch_dense(p, parts, s);
+        if (st != AKAS_OK) return st;
+      } else if (scale_dtype == AKAS_DTYPE_F32) {
         launch_split_m<1, AKAS_DTYPE_F32, AKAS_DTYPE_F32>(p, parts, s);
-      else
+      } else {
         launch_split_m<1, AKAS_DTYPE_F32, AKAS_DTYPE_BF16>(p, parts, s);
+      }
       const int64_t n = r * o, want = (n + 255) / 256;
       merge_kernel<<<(int)(want < 16384 ? want : 16384), 256, 0, s>>>(partial, out, out_dtype, r, o,
                                                                        parts);
