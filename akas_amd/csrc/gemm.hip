@@ -579,6 +579,7 @@ __global__ __launch_bounds__(E::THREADS) void dense_pipe_kernel(DenseArgs p) {
 
   typename E::Acc acc;
   acc.clear();
+  e.start(plan, kb0, nkb);
   e.template run<false>(plan, acc, kb0, nkb, [&](int kb) {
     const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kb < 64 ? wreg[0] : wreg[1]), kb & 63));
     return float2{w, w};

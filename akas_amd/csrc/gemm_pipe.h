@@ -129,21 +129,50 @@ struct Engine {
 
   // The DMA of step t into stage S: the group's k-block, clamped to the last
   // (a clamped copy is never multiplied).  plan.a(i, kb) / plan.b(i, kb) are
-  // the addresses of this lane's 16 bytes of piece i, plan.s(kb) that of its scale.
+  // the addresses of this lane's 16 bytes of piece i, plan.s(kb) that of its
+  // scale.
   template <int S, class Plan>
-  AKAS_DEV void issue(const Plan& plan, int t, int kb0, int nkb) const {
+  AKAS_DEV void issue_a(const Plan& plan, int t, int kb0, int nkb) const {
     const int kb = kb0 + min(t * G + g, nkb - 1);
     uint8_t* base = stage<S>() + g * TILE;
 #pragma unroll
     for (int i = 0; i < PA; ++i)
       __builtin_amdgcn_global_load_lds((const void*)plan.a(i, kb),
                                        (lds_void*)(base + (w * PA + i) * 1024), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((const void*)plan.s(kb),
+                                     (lds_void*)(stage_scales<S>() + g * BM + (w % SR) * 64), 4, 0, 0);
+  }
+  template <int S, class Plan>
+  AKAS_DEV void issue_b(const Plan& plan, int t, int kb0, int nkb) const {
+    const int kb = kb0 + min(t * G + g, nkb - 1);
+    uint8_t* base = stage<S>() + g * TILE + BM * 128;
 #pragma unroll
     for (int i = 0; i < PB; ++i)
       __builtin_amdgcn_global_load_lds((const void*)plan.b(i, kb),
-                                       (lds_void*)(base + BM * 128 + (w * PB + i) * 1024), 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((const void*)plan.s(kb),
-                                     (lds_void*)(stage_scales<S>() + g * BM + (w % SR) * 64), 4, 0, 0);
+                                       (lds_void*)(base + (w * PB + i) * 1024), 16, 0, 0);
+  }
+  template <int S, class Plan>
+  AKAS_DEV void issue(const Plan& plan, int t, int kb0, int nkb) const {
+    issue_a<S>(plan, t, kb0, nkb);
+    issue_b<S>(plan, t, kb0, nkb);
+  }
+
+  // The stages ahead of the first step, B (known first where A rows are
+  // gathered through a table) and A; then wait until stage 0 has landed.
+  template <class Plan>
+  AKAS_DEV void start_b(const Plan& plan, int kb0, int nkb) const {
+    issue_b<0>(plan, 0, kb0, nkb);
+    if constexpr (AHEAD > 1) issue_b<1>(plan, 1, kb0, nkb);
+    if constexpr (AHEAD > 2) issue_b<2>(plan, 2, kb0, nkb);
+  }
+  template <class Plan>
+  AKAS_DEV void start_a(const Plan& plan, int kb0, int nkb) const {
+    issue_a<0>(plan, 0, kb0, nkb);
+    if constexpr (AHEAD > 1) issue_a<1>(plan, 1, kb0, nkb);
+    if constexpr (AHEAD > 2) issue_a<2>(plan, 2, kb0, nkb);
+    // (deeper, run's constant waits would count a younger stage's B as A)
+    static_assert(AHEAD <= 2, "B ahead of A: two stages at most");
+    wait_loads<(PA + 1) * (AHEAD - 1)>();
   }
 
   // One k-block of stage S into acc: acc = fma(P, as * ws, acc) per product.
@@ -182,40 +211,46 @@ struct Engine {
   // landed and that every wave is done with the stage that is refilled.
   // FULL steps all issue a stage, so their wait is a constant.
   template <int S, bool FULL, bool PAIRED, class Plan, class WS>
-  AKAS_DEV void step(const Plan& plan, Acc& acc, int t, int steps, int kb0, int nkb, WS ws) const {
+  AKAS_DEV void step(const Plan& plan, Acc& acc, int t, int steps, int kb0, int nkb, WS ws,
+                     bool live) const {
     wait_loads<FULL ? LOADS * (AHEAD - 1) : 0>();
     barrier();
     if (FULL || t + AHEAD < steps) issue<(S + AHEAD) % ST>(plan, t + AHEAD, kb0, nkb);
     const int kb = t * G + g;
-    if (G == 1 || kb < nkb) {
+    if (live && (G == 1 || kb < nkb)) {
       const float2 v = ws(kb);
       multiply<S, PAIRED>(acc, v.x, v.y);
     }
   }
 
-  // k-blocks [kb0, kb0 + nkb) into acc.  ws(i) is the (ws0, ws1) pair of
-  // k-block kb0 + i; it must come from registers (a global or LDS load there
-  // would wait for the copies in flight).
-  template <bool PAIRED, class Plan, class WS>
-  AKAS_DEV void run(const Plan& plan, Acc& acc, int kb0, int nkb, WS ws) const {
-    const int steps = (nkb + G - 1) / G;
+  // k-blocks [kb0, kb0 + nkb) into acc, after start_b and start_a (or
+  // start).  ws(i) is the (ws0, ws1) pair of k-block kb0 + i; it must come
+  // from registers (a global or LDS load there would wait for the copies in
+  // flight).  A wave that is not `live` only copies: no row or column of its
+  // tile is stored.
+  template <class Plan>
+  AKAS_DEV void start(const Plan& plan, int kb0, int nkb) const {
     issue<0>(plan, 0, kb0, nkb);
     if constexpr (AHEAD > 1) issue<1>(plan, 1, kb0, nkb);
     if constexpr (AHEAD > 2) issue<2>(plan, 2, kb0, nkb);
+  }
+  template <bool PAIRED, class Plan, class WS>
+  AKAS_DEV void run(const Plan& plan, Acc& acc, int kb0, int nkb, WS ws, bool live = true) const {
+    const int steps = (nkb + G - 1) / G;
     int t = 0;
     for (; t + ST + AHEAD <= steps; t += ST) {
-      step<0, true, PAIRED>(plan, acc, t, steps, kb0, nkb, ws);
-      step<1, true, PAIRED>(plan, acc, t + 1, steps, kb0, nkb, ws);
-      if constexpr (ST > 2) step<2, true, PAIRED>(plan, acc, t + 2, steps, kb0, nkb, ws);
-      if constexpr (ST > 3) step<3, true, PAIRED>(plan, acc, t + 3, steps, kb0, nkb, ws);
+      step<0, true, PAIRED>(plan, acc, t, steps, kb0, nkb, ws, live);
+      step<1, true, PAIRED>(plan, acc, t + 1, steps, kb0, nkb, ws, live);
+      if constexpr (ST > 2) step<2, true, PAIRED>(plan, acc, t + 2, steps, kb0, nkb, ws, live);
+      if constexpr (ST > 3) step<3, true, PAIRED>(plan, acc, t + 3, steps, kb0, nkb, ws, live);
     }
     for (; t < steps; t += ST) {
-      step<0, false, PAIRED>(plan, acc, t, steps, kb0, nkb, ws);
-      if (t + 1 < steps) step<1, false, PAIRED>(plan, acc, t + 1, steps, kb0, nkb, ws);
+      step<0, false, PAIRED>(plan, acc, t, steps, kb0, nkb, ws, live);
+      if (t + 1 < steps) step<1, false, PAIRED>(plan, acc, t + 1, steps, kb0, nkb, ws, live);
       if constexpr (ST > 2)
-        if (t + 2 < steps) step<2, false, PAIRED>(plan, acc, t + 2, steps, kb0, nkb, ws);
+        if (t + 2 < steps) step<2, false, PAIRED>(plan, acc, t + 2, steps, kb0, nkb, ws, live);
       if constexpr (ST > 3)
-        if (t + 3 < steps) step<3, false, PAIRED>(plan, acc, t + 3, steps, kb0, nkb, ws);
+        if (t + 3 < steps) step<3, false, PAIRED>(plan, acc, t + 3, steps, kb0, nkb, ws, live);
     }
   }
 
@@ -224,7 +259,6 @@ struct Engine {
   // c ^ (r & SWZ), conflict-free for the accumulators' writes and for row reads.
   static constexpr int TILE_F32 = TM * TN * 4, PER_STAGE = STAGE / TILE_F32;
   static constexpr int SWZ = TN / 4 >= 16 ? 15 : TN / 4 - 1;
-  static_assert(PER_STAGE * ST >= W * G, "the partial tiles fit in the stages");
   AKAS_DEV uint8_t* partial(int q) const {
     const int slot = q * W + w, s = slot / PER_STAGE;
     uint8_t* base = stage<0>();
@@ -239,6 +273,7 @@ struct Engine {
   // and col relative to the workgroup's tile.  The groups share the pieces.
   template <class Put>
   AKAS_DEV void reduce(const Acc& acc, Put put) const {
+    static_assert(PER_STAGE * ST >= W * G, "the partial tiles fit in the stages");
     __syncthreads();  // the stages are read no more, and no copy is in flight
     uint8_t* own = partial(g);
 #pragma unroll

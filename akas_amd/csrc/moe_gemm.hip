@@ -22,6 +22,7 @@
 #include "device_info.h"
 #include "gemm_core.h"
 #include "gemm_dma.h"
+#include "gemm_pipe.h"
 #include "moe_launch.h"
 #include "quant_group.h"
 
@@ -958,6 +959,196 @@ __global__ __launch_bounds__(dma::THREADS) void expert_dma_kernel(ExpertArgs p) 
 }
 
 // ---------------------------------------------------------------------------
+// Experts of about fifty to a hundred rows each, on the pipelined engine
+// (gemm_pipe.h) with one k-block group, so every (row, column) is still one
+// f32 chain in ascending k-block order and the results are those of the other
+// grouped kernels bit for bit.  Modes kPartial and kSwigluFp8.
+//
+// These batches read every expert's weights for one or two row tiles, so the
+// bound is HBM; register-staged 128-row tiles keep one k-block per workgroup
+// in flight.  64 experts x 1536 x 2048, bf16 intermediates, GEMMs alone in
+// us: gate/up 111.8 -> 95.7 at 900 tokens x 4, 112.1 -> 104.3 at 1500; down
+// 45.3 -> 41.1, 47.7 -> 44.9.  The first stages' weights are requested before
+// the tile's rows are known.  (Chaining a workgroup's items, the next one's
+// weights requested under the epilogue, measured 98.7 / 107.6: the load rate
+// inside the k-loop, not the gaps between tiles, is what holds them.)
+// ---------------------------------------------------------------------------
+constexpr int kExpertPipeMaxKb = 128;
+
+struct ExpertPipePlan {
+  const uint8_t* a_base;
+  const uint8_t* b_base;
+  const float* as;
+  int64_t alt_delta;   // added for the pieces of alt_mask (the up bank)
+  uint32_t alt_mask;   // wave-uniform
+  uint32_t a_off[4], b_off[4], s_off;
+  AKAS_DEV const uint8_t* a(int i, int kb) const { return a_base + (int64_t)kb * kBlock + a_off[i]; }
+  AKAS_DEV const uint8_t* b(int i, int kb) const {
+    const int64_t bank = ((alt_mask >> i) & 1u) ? alt_delta : 0;
+    return b_base + (bank + (int64_t)kb * kBlock + b_off[i]);
+  }
+  AKAS_DEV const float* s(int kb) const { return as + kb + s_off; }
+};
+
+template <class E, int MODE, int OUT, int SDT>
+__global__ __launch_bounds__(E::THREADS) void expert_pipe_kernel(ExpertArgs p) {
+  constexpr bool PAIRED = paired_mode(MODE);
+  constexpr int BM = E::BM, WAVES_N = E::BN / E::TN;
+  static_assert(E::G == 1 && (MODE == kPartial || MODE == kSwigluFp8), "one k-block group");
+  static_assert(!PAIRED || E::BN == 256, "paired tiles hold 128 gate + 128 up");
+  static_assert(BM <= E::THREADS && E::PA <= 4 && E::PB <= 4, "table and plan sizes");
+  __shared__ int rows_dst[BM];
+  __shared__ float row_max[PAIRED ? WAVES_N : 1][PAIRED ? BM : 1];
+
+  const int tid = threadIdx.x;
+  const E eng(tid);
+  const int lane = eng.lane;
+  Item item;
+  if (!find_item(p.counts, p.E, p.r, BM, p.tiles_n, lane, item)) return;  // uniform
+  const int e = item.expert, count = item.count, row0 = item.tile * BM;
+  if (row0 >= count) return;  // only reachable with counts[e] > r
+  const int n0 = item.nb * (PAIRED ? E::BN / 2 : E::BN);
+  const int KB = p.K / kBlock, NB = (p.N + kBlock - 1) / kBlock;
+  const int part = blockIdx.y, nkb = p.kb_per_part, kb0 = part * nkb;
+  const ExpertSlice xs = expert_slice(p, e);
+  // First output column of this wave; gate and up share its scale block.
+  const int wcol = PAIRED ? n0 + eng.b_row0 / 2 : n0 + eng.b_row0;
+
+  // Loads that need only the item: the routes of the rows this thread
+  // copies, scales and scatters, the weight scales (lane l: k-blocks l and
+  // 64 + l), then the weights of the first stages.
+  const auto index = [&](int row) { return row0 + row < count ? row0 + row : row0; };
+  RowRoute qa[E::PA], qs, qd{0, 0};
+#pragma unroll
+  for (int i = 0; i < E::PA; ++i) qa[i] = tile_route(p, e, index(eng.a_piece_row(i)));
+  qs = tile_route(p, e, index(eng.scale_row()));
+  if (tid < BM) qd = tile_route(p, e, index(tid));
+  uint32_t wraw[2][2];
+  {
+    const int64_t base = ((int64_t)xs.scale_expert * NB + wcol / kBlock) * KB + kb0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t at = base + min(lane + 64 * h, nkb - 1);
+#pragma unroll
+      for (int u = 0; u < (PAIRED ? 2 : 1); ++u) {
+        const void* src = u ? xs.ws2 : xs.ws;
+        wraw[u][h] = SDT == AKAS_DTYPE_F32 ? reinterpret_cast<const uint32_t*>(src)[at]
+                                           : reinterpret_cast<const uint16_t*>(src)[at];
+      }
+    }
+  }
+  ExpertPipePlan plan;
+  plan.a_base = p.x;
+  plan.b_base = xs.w;
+  plan.as = p.as;
+  plan.alt_delta = PAIRED ? (int64_t)(xs.w2 - xs.w) : 0;
+  plan.alt_mask = 0;
+#pragma unroll
+  for (int i = 0; i < E::PB; ++i) {
+    const int rho = eng.b_piece_row(i);
+    // PAIRED: 16-row tile rho / 16 is gate (even) or up (odd)
+    if (PAIRED) plan.alt_mask |= (uint32_t)(((eng.w * E::PB + i) >> 1) & 1) << i;
+    const int col = PAIRED ? n0 + (rho >> 5) * 16 + (rho & 15) : n0 + rho;
+    plan.b_off[i] = (uint32_t)col * (uint32_t)p.K + eng.piece_chunk(rho);
+  }
+  eng.start_b(plan, kb0, nkb);
+
+  int src, dst;
+#pragma unroll
+  for (int i = 0; i < E::PA; ++i) {
+    const int row = eng.a_piece_row(i);
+    tile_row_of(p, qa[i], index(row), false, src, dst);
+    plan.a_off[i] = (uint32_t)src * (uint32_t)p.K + eng.piece_chunk(row);
+  }
+  tile_row_of(p, qs, index(eng.scale_row()), false, src, dst);
+  plan.s_off = (uint32_t)src * (uint32_t)KB;
+  if (tid < BM) {
+    tile_row_of(p, qd, index(tid), row0 + tid < count, src, dst);
+    rows_dst[tid] = dst;
+  }
+  float wreg[2][2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t raw = wraw[PAIRED ? u : 0][h];
+      wreg[u][h] = __uint_as_float(SDT == AKAS_DTYPE_F32 ? raw : raw << 16);
+    }
+  eng.start_a(plan, kb0, nkb);
+
+  typename E::Acc acc;
+  acc.clear();
+  const auto scale = [&](int u, int kb) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(kb < 64 ? wreg[u][0] : wreg[u][1]), kb & 63));
+  };
+  eng.template run<PAIRED>(plan, acc, kb0, nkb, [&](int kb) {
+    const float g = scale(0, kb);
+    return float2{g, PAIRED ? scale(1, kb) : g};
+  }, row0 + eng.a_row0 < count);  // a wave whose rows are all padding only copies
+
+  if constexpr (!PAIRED) {
+    const int64_t rstride = (int64_t)p.parts * p.N;
+    const bool wide = reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
+    eng.reduce(acc, [&](int row, int col, const v4f& lo, const v4f& hi) {
+      const int d = rows_dst[row];
+      if (d >= 0)
+        pipe::store_out8<OUT>(p.out, (int64_t)d * rstride + (int64_t)part * p.N + n0 + col, lo, hi, wide);
+    });
+  } else {
+    // Lane l holds, for row tile i and column group c, gate in 16-column
+    // tile 2c and up in 2c + 1 of row a_row0 + 16i + l % 16 at output columns
+    // wcol + 16c + 4 * (l / 16) .. +3.  SwiGLU in place of the gate values,
+    // then the row maximum over the tile's 128 output columns.
+    const int wn = eng.b_row0 / E::TN;
+    float rmax[E::MT];
+    with_dtype(p.prod_dtype, [&](auto PD) __attribute__((always_inline)) {
+      with_dtype(p.act_dtype, [&](auto AD) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < E::MT; ++i) {
+          float m = 0.f;
+#pragma unroll
+          for (int c = 0; c < E::NT / 2; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const float g = round_t<decltype(PD)::value>(acc.t[i][2 * c][q]);
+              const float u = round_t<decltype(PD)::value>(acc.t[i][2 * c + 1][q]);
+              const float a = round_t<decltype(AD)::value>(swiglu_elem(g, u));
+              acc.t[i][2 * c][q] = a;
+              m = __builtin_fmaxf(m, __builtin_fabsf(a));
+            }
+          rmax[i] = m;
+        }
+      });
+    });
+#pragma unroll
+    for (int i = 0; i < E::MT; ++i) {
+      float m = __builtin_fmaxf(rmax[i], __shfl_xor(rmax[i], 16, 64));
+      m = __builtin_fmaxf(m, __shfl_xor(m, 32, 64));
+      if (lane < 16) row_max[wn][eng.a_row0 + 16 * i + lane] = m;
+    }
+    __syncthreads();
+    uint8_t* codes = reinterpret_cast<uint8_t*>(p.out);
+#pragma unroll
+    for (int i = 0; i < E::MT; ++i) {
+      const int r = eng.a_row0 + 16 * i + (lane & 15);
+      float m = row_max[0][r];
+#pragma unroll
+      for (int w = 1; w < WAVES_N; ++w) m = __builtin_fmaxf(m, row_max[w][r]);
+      const GroupScale gs = make_group_scale(m);
+      const int d = rows_dst[r];
+      if (d < 0) continue;
+#pragma unroll
+      for (int c = 0; c < E::NT / 2; ++c) {
+        const v4f& a = acc.t[i][2 * c];
+        *reinterpret_cast<uint32_t*>(codes + (int64_t)d * p.N + wcol + 16 * c + 4 * (lane >> 4)) =
+            e4m3_encode4_scaled(a[0], a[1], a[2], a[3], gs);
+      }
+      if (wn == 0 && lane < 16) p.out_scales[(int64_t)d * (p.N / kBlock) + n0 / kBlock] = gs.s;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // fp8_experts' group tables (moe_groups: experts [r*top], routes [r*top, r]
 // holding a rank or -1) -> the grouped kernels' per-expert counts and routes
 // (row*top + rank, in row order).  One workgroup per expert finds the group
@@ -1027,6 +1218,17 @@ static void launch_expert(ExpertArgs a, hipStream_t s) {
         <<<grid, 64 * WMW * WNW, 0, s>>>(a);
 }
 
+template <class E, int MODE, int OUT>
+static void launch_expert_pipe(ExpertArgs a, hipStream_t s) {
+  a.max_tiles = (int)capacity_tiles(a.r, a.top, a.E, E::BM);
+  a.tiles_n = paired_mode(MODE) ? a.N / (E::BN / 2) : a.N / E::BN;
+  dim3 grid((unsigned)(a.max_tiles * a.tiles_n), (unsigned)a.parts);
+  if (a.ws_dtype == AKAS_DTYPE_F32)
+    expert_pipe_kernel<E, MODE, OUT, AKAS_DTYPE_F32><<<grid, E::THREADS, 0, s>>>(a);
+  else
+    expert_pipe_kernel<E, MODE, OUT, AKAS_DTYPE_BF16><<<grid, E::THREADS, 0, s>>>(a);
+}
+
 template <int MODE, int OUT>
 static void launch_expert_dma(ExpertArgs a, hipStream_t s) {
   a.max_tiles = (int)capacity_tiles(a.r, a.top, a.E, dma::BM);
@@ -1035,18 +1237,47 @@ static void launch_expert_dma(ExpertArgs a, hipStream_t s) {
   expert_dma_kernel<MODE, OUT><<<grid, dma::THREADS, 0, s>>>(a);
 }
 
-// Experts holding hundreds of rows on average (prefill batches) take the
-// DMA-fed 256-row tiles; its 16-byte stores need a 16-byte aligned output.
-static bool expert_dma_fits(const ExpertArgs& a, int64_t mean, int64_t n_mult) {
-  return mean >= 128 && a.N % n_mult == 0 && a.kb_per_part <= dma::MAX_KB &&
+// The DMA-fed 256-row tiles (prefill batches); its 16-byte stores need a
+// 16-byte aligned output.
+static bool expert_dma_fits(const ExpertArgs& a, int64_t n_mult) {
+  return a.N % n_mult == 0 && a.kb_per_part <= dma::MAX_KB &&
          reinterpret_cast<uintptr_t>(a.out) % 16 == 0;
 }
 
-// Row tile by the mean rows per expert: 32-row tiles for decode-like batches,
-// 128-row tiles in between, DMA-fed 256-row tiles for prefill batches.
+// The pipelined engine's DMA takes 16-byte aligned codes (rows are multiples
+// of 128 bytes).
+static bool expert_pipe_fits(const ExpertArgs& a) {
+  const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  return a.kb_per_part <= kExpertPipeMaxKb && aligned(a.x) && aligned(a.w) && aligned(a.w2) &&
+         aligned(a.xw) && aligned(a.xw2);
+}
+
+// Row tile by the mean rows per expert (the down projection of 64 experts,
+// 1536 -> 2048, us):
+//   below 32     32-row tiles (mean 16: 40; 25: 41.4, 35.6 on the next)
+//   32 to 64     64-row pipelined tiles, three workgroups per CU (mean 40:
+//                45.7 -> 36.8; 128 experts, 512 -> 2048, mean 44: 35.8 ->
+//                33.5, but mean 25: 29.9, 31.5 on 64 rows)
+//   to 111       128-row pipelined tiles, two per CU (mean 94: 47.7 -> 44.9)
+//   beyond       DMA-fed 256-row tiles (mean 125: 53.0 against 58.1; 94: 51.4
+//                against 44.9)
+// expert_combine, and codes off the pipelined engine's alignment, keep
+// 32-row tiles to a mean of 48 and register-staged 128-row tiles after.
 template <int OUT, int MODE = kPartial>
 static void launch_partial(const ExpertArgs& a, hipStream_t s) {
   const int64_t mean = (int64_t)a.r * a.top / a.E;
+  const bool piped = MODE == kPartial && mean >= 32 && expert_pipe_fits(a);
+  if (mean >= 112 && expert_dma_fits(a, dma::BN)) {
+    launch_expert_dma<MODE, OUT>(a, s);
+    return;
+  }
+  if constexpr (MODE == kPartial) {
+    if (piped && mean <= 64)
+      launch_expert_pipe<pipe::Engine<64, 128, 2, 2, 1, 2>, MODE, OUT>(a, s);
+    else if (piped)
+      launch_expert_pipe<pipe::Engine<128, 128, 2, 2, 1, 2>, MODE, OUT>(a, s);
+  }
+  if (piped) return;
   // 256-column tiles where N allows: half the workgroups of 128-column ones,
   // each streaming twice the weights (LFM2 decode layer 146.0 -> 145.0 us,
   // the Qwen3.5 block 191.9 -> 189.2 us; 512 columns was slower).
@@ -1054,8 +1285,6 @@ static void launch_partial(const ExpertArgs& a, hipStream_t s) {
     launch_expert<32, 256, 1, 4, MODE, OUT>(a, s);
   else if (mean <= 48)
     launch_expert<32, 128, 1, 4, MODE, OUT>(a, s);
-  else if (expert_dma_fits(a, mean, dma::BN))
-    launch_expert_dma<MODE, OUT>(a, s);
   else
     launch_expert<128, 128, 2, 2, MODE, OUT>(a, s);
 }
@@ -1066,6 +1295,7 @@ static void launch_partial(const ExpertArgs& a, hipStream_t s) {
 template <int MODE, int OUT, int SCAN = 0>
 static void launch_paired(const ExpertArgs& a, hipStream_t s) {
   const int64_t mean = (int64_t)a.r * a.top / a.E;
+  const int64_t cus = device_cus();
   const bool aligned = MODE != kPairPartial || reinterpret_cast<uintptr_t>(a.out2) % 16 == 0;
   // Decode batches: about one 32-row tile per active expert, at most
   // min(E, r*top) of them per column block.  When all of those workgroups fit
@@ -1074,23 +1304,40 @@ static void launch_paired(const ExpertArgs& a, hipStream_t s) {
   // 135.5 us); when they do not, the two-stage tile's faster workgroups win
   // (Qwen3.5 block, about 900 workgroups: 184.0 against 191.4 us one-stage).
   const int64_t decode_tiles = std::min<int64_t>(a.E, (int64_t)a.r * a.top) * (a.N / 128) * a.parts;
-  if (mean <= 8 && decode_tiles <= 4 * (int64_t)device_cus() + device_cus() / 4) {
+  if (mean <= 8 && decode_tiles <= 4 * cus + cus / 4) {
     // a few rows per expert: 16-row tiles, four workgroups per CU
     ExpertArgs b = a;
-    b.fair = decode_tiles >= 2 * (int64_t)device_cus();
+    b.fair = decode_tiles >= 2 * cus;
     launch_expert<16, 256, 1, 4, MODE, OUT, 1, SCAN>(b, s);
-  } else if (mean <= 48 && decode_tiles <= 3 * (int64_t)device_cus()) {
+  } else if (mean <= 48 && decode_tiles <= 3 * cus) {
     // one round: progress-ordered priority once workgroups share CUs
     ExpertArgs b = a;
-    b.fair = decode_tiles >= 2 * (int64_t)device_cus();
+    b.fair = decode_tiles >= 2 * cus;
     launch_expert<32, 256, 1, 4, MODE, OUT, 1, SCAN>(b, s);
   } else if (mean <= 48) {
     launch_expert<32, 256, 1, 4, MODE, OUT, 0, SCAN>(a, s);
   } else if constexpr (!SCAN) {
-    if (aligned && expert_dma_fits(a, mean, dma::BN / 2))
+    // Above 48 mean rows: the DMA-fed 256-row tiles from a mean of 100 (64
+    // experts, 2048 -> 1536: mean 106 121.6 us against 132.0 on 128 rows; 94:
+    // 121 against 104.3), unless too few of them for the CUs and one or two
+    // 128-row tiles hold an expert (32 experts, 1024 -> 512, mean 175: 26.7,
+    // 24.5; 275: 28.7, 39.7).  Before, the pipelined 128-row tile, or its
+    // 64-row one while 128-row tiles would leave CUs idle (the same 32
+    // experts, mean 62: 22.0 register-staged, 18.9 on 128 rows, 15.3 on 64).
+    const int64_t column_blocks = a.N / 128 * a.parts;
+    const bool few = (int64_t)a.E * ((mean + 255) / 256) * column_blocks < cus * 3 / 4;
+    const bool piped = MODE == kSwigluFp8 && expert_pipe_fits(a);
+    if (aligned && mean >= 100 && !(piped && few && mean <= 240) && expert_dma_fits(a, dma::BN / 2)) {
       launch_expert_dma<MODE, OUT>(a, s);
-    else
-      launch_expert<128, 256, 2, 4, MODE, OUT>(a, s);
+      return;
+    }
+    if constexpr (MODE == kSwigluFp8) {
+      if (piped && mean <= 64 && a.E * column_blocks < cus)
+        launch_expert_pipe<pipe::Engine<64, 256, 2, 4, 1, 3>, MODE, OUT>(a, s);
+      else if (piped)
+        launch_expert_pipe<pipe::Engine<128, 256, 2, 4, 1, 3>, MODE, OUT>(a, s);
+    }
+    if (!piped) launch_expert<128, 256, 2, 4, MODE, OUT>(a, s);
   }
 }
 
