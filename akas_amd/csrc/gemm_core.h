@@ -35,7 +35,9 @@ AKAS_DEV int lds_off(int row, int chunk) { return row * 128 + ((chunk ^ ((row & 
 // the loads use scalar-base addressing with one VGPR per address.  Rows past the end of an operand are clamped to a valid row
 // by the caller: their products land in rows/columns that are never stored
 // or carry a zero scale, so no branch is needed in the copy loop.
-template <int BM, int BN, int THREADS>
+// STREAM: B (the weights) is loaded with the non-temporal hint, for weights
+// that this launch reads once and from HBM.
+template <int BM, int BN, int THREADS, bool STREAM = false>
 struct StagePlan {
   static constexpr int RSTEP = THREADS / 8;
   // A_PART: fewer A rows than thread rows (a 16-row tile on 256 threads):
@@ -66,8 +68,10 @@ struct StagePlan {
   AKAS_DEV void fetch_b(int kb, u32x4 (&rb)[CB]) const {
     const uint32_t ko = (uint32_t)kb * kBlock;
 #pragma unroll
-    for (int j = 0; j < CB; ++j)
-      rb[j] = *reinterpret_cast<const u32x4*>(b_base + (b_off + j * b_step + ko));
+    for (int j = 0; j < CB; ++j) {
+      const u32x4* src = reinterpret_cast<const u32x4*>(b_base + (b_off + j * b_step + ko));
+      rb[j] = STREAM ? __builtin_nontemporal_load(src) : *src;
+    }
   }
   AKAS_DEV void fetch(int kb, u32x4 (&ra)[CA], u32x4 (&rb)[CB]) const {
     fetch_a(kb, ra);

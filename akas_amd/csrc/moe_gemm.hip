@@ -466,8 +466,9 @@ AKAS_DEV void wave_priority_by_progress(int done, int total) {
 // SIMD, so that three workgroups share a CU.
 // SCAN: the workgroup scans ids itself (scan_entries) instead of reading the
 // route tables, and writes them for the launches after it.
+// STREAM: the weights take non-temporal loads (see stream_weights).
 template <int BM, int BN, int WAVES_M, int WAVES_N, int MODE, int OUT, int SDT, int STAGES = 0,
-          int SCAN = 0>
+          int SCAN = 0, bool STREAM = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N)
 __attribute__((amdgpu_waves_per_eu((STAGES == 1 && BM == 16 && paired_mode(MODE)) ? 4
                                    : (STAGES == 1 && BM == 32 && paired_mode(MODE)) ? 3 : 1)))
@@ -478,7 +479,7 @@ void expert_tiled_kernel(ExpertArgs p) {
   constexpr bool PAIRED = paired_mode(MODE);
   static_assert(!PAIRED || (BN == 256 && NT % 2 == 0), "paired tiles hold 128 gate + 128 up");
   static_assert(PAIRED || 128 % WN == 0, "a wave's columns must stay inside one scale block");
-  using Plan = StagePlan<BM, BN, THREADS>;
+  using Plan = StagePlan<BM, BN, THREADS, STREAM>;
   constexpr int STAGE = (BM + BN) * 128;
   // The 32-row expert partial (the decode down projection) keeps one LDS
   // stage, so that more workgroups share a CU: four instead of three with
@@ -1205,17 +1206,46 @@ int64_t capacity_tiles(int64_t r, int64_t top, int64_t experts, int64_t bm) {
   return routes < b ? routes : b;
 }
 
-template <int BM, int BN, int WMW, int WNW, int MODE, int OUT, int STAGES = 0, int SCAN = 0>
+template <int BM, int BN, int WMW, int WNW, int MODE, int OUT, int STAGES = 0, int SCAN = 0,
+          bool STREAM = false>
 static void launch_expert(ExpertArgs a, hipStream_t s) {
   a.max_tiles = (int)capacity_tiles(a.r, a.top, a.E, BM);
   a.tiles_n = paired_mode(MODE) ? a.N / (BN / 2) : a.N / BN;
   dim3 grid((unsigned)(a.max_tiles * a.tiles_n), (unsigned)a.parts);
   if (a.ws_dtype == AKAS_DTYPE_F32)
-    expert_tiled_kernel<BM, BN, WMW, WNW, MODE, OUT, AKAS_DTYPE_F32, STAGES, SCAN>
+    expert_tiled_kernel<BM, BN, WMW, WNW, MODE, OUT, AKAS_DTYPE_F32, STAGES, SCAN, STREAM>
         <<<grid, 64 * WMW * WNW, 0, s>>>(a);
   else
-    expert_tiled_kernel<BM, BN, WMW, WNW, MODE, OUT, AKAS_DTYPE_BF16, STAGES, SCAN>
+    expert_tiled_kernel<BM, BN, WMW, WNW, MODE, OUT, AKAS_DTYPE_BF16, STAGES, SCAN, STREAM>
         <<<grid, 64 * WMW * WNW, 0, s>>>(a);
+}
+
+// Whether a decode launch loads its weights with the non-temporal hint: when
+// it streams at least 96 MB of them, more than a call can leave in the 256 MB
+// last-level cache for the next, and most experts have one row tile, so that
+// no second tile reads them again.  Without the hint every line streamed
+// displaces another from the caches on its way (64 experts, 2048 -> 1536 ->
+// 2048, whole block: 256 tokens 131.3 -> 122.4 us, 64 125.6 -> 116.1, 400
+// 166.4 -> 158.9; 256 experts of 512 and a shared one, 64 tokens 157.8 ->
+// 152.5).  With two row tiles per expert it loses (640 tokens 160.4 -> 180.7),
+// and with weights that stay in the cache from call to call (32 experts, 1024
+// -> 512, 64 tokens: 31.6 -> 35.0).
+static bool stream_weights(const ExpertArgs& a, int64_t bytes_per_expert) {
+  const int64_t routes = (int64_t)a.r * a.top;
+  return std::min<int64_t>(a.E, routes) * bytes_per_expert >= (96ll << 20) && routes / a.E <= 28;
+}
+
+// A decode launch with or without the hint (the modes that decode runs).
+template <int BM, int BN, int MODE, int OUT, int STAGES = 0, int SCAN = 0>
+static void launch_decode_expert(const ExpertArgs& a, hipStream_t s) {
+  if constexpr (MODE == kPartial || MODE == kSwigluFp8) {
+    const int64_t bytes = (int64_t)a.N * a.K * (paired_mode(MODE) ? 2 : 1);
+    if (stream_weights(a, bytes)) {
+      launch_expert<BM, BN, 1, 4, MODE, OUT, STAGES, SCAN, true>(a, s);
+      return;
+    }
+  }
+  launch_expert<BM, BN, 1, 4, MODE, OUT, STAGES, SCAN>(a, s);
 }
 
 template <class E, int MODE, int OUT>
@@ -1282,7 +1312,7 @@ static void launch_partial(const ExpertArgs& a, hipStream_t s) {
   // each streaming twice the weights (LFM2 decode layer 146.0 -> 145.0 us,
   // the Qwen3.5 block 191.9 -> 189.2 us; 512 columns was slower).
   if (mean <= 48 && a.N % 256 == 0)
-    launch_expert<32, 256, 1, 4, MODE, OUT>(a, s);
+    launch_decode_expert<32, 256, MODE, OUT>(a, s);
   else if (mean <= 48)
     launch_expert<32, 128, 1, 4, MODE, OUT>(a, s);
   else
@@ -1308,14 +1338,14 @@ static void launch_paired(const ExpertArgs& a, hipStream_t s) {
     // a few rows per expert: 16-row tiles, four workgroups per CU
     ExpertArgs b = a;
     b.fair = decode_tiles >= 2 * cus;
-    launch_expert<16, 256, 1, 4, MODE, OUT, 1, SCAN>(b, s);
+    launch_decode_expert<16, 256, MODE, OUT, 1, SCAN>(b, s);
   } else if (mean <= 48 && decode_tiles <= 3 * cus) {
     // one round: progress-ordered priority once workgroups share CUs
     ExpertArgs b = a;
     b.fair = decode_tiles >= 2 * cus;
-    launch_expert<32, 256, 1, 4, MODE, OUT, 1, SCAN>(b, s);
+    launch_decode_expert<32, 256, MODE, OUT, 1, SCAN>(b, s);
   } else if (mean <= 48) {
-    launch_expert<32, 256, 1, 4, MODE, OUT, 0, SCAN>(a, s);
+    launch_decode_expert<32, 256, MODE, OUT, 0, SCAN>(a, s);
   } else if constexpr (!SCAN) {
     // Above 48 mean rows: the DMA-fed 256-row tiles from a mean of 100 (64
     // experts, 2048 -> 1536: mean 106 121.6 us against 132.0 on 128 rows; 94:
