@@ -708,7 +708,6 @@ __global__ __launch_bounds__(256) void dense_small_kernel(DenseArgs p) {
 // Weights stream from HBM exactly once; activations are read from L2 once
 // per workgroup instead of once per wave.
 // ---------------------------------------------------------------------------
-constexpr int kWideBatch = 2;  // k-blocks of weights in flight per wave
 
 template <int MT, int NTW, int KS>
 constexpr size_t wide_lds_bytes(int kbp) {
@@ -731,7 +730,13 @@ constexpr size_t wide_lds_bytes(int kbp) {
 // count: at N = 6144, 24 columns give 256 workgroups where 32 give 192.
 // A 24-column workgroup loads its weight scales per lane (its tiles can
 // straddle a 128-column scale block).
-template <int MT, int NTW, int KS, int OUT, int SDT, int QX = 0, int CW = 16 * NTW>
+//
+// B: k-blocks of weights in flight per wave.  Two cover a 2048-deep product
+// (16 k-blocks over KS = 8 waves); deeper ones take four or eight: in batches
+// of two, each batch waited a memory round trip for its own loads (fp8_linear
+// M=1, K=8192, N=2048 9.2 -> 8.2 us; at K=2048 eight slots lose, N=6144 5.3 ->
+// 6.1).
+template <int MT, int NTW, int KS, int OUT, int SDT, int QX = 0, int CW = 16 * NTW, int B = 2>
 __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) {
   static_assert(CW > 16 * (NTW - 1) && CW <= 16 * NTW, "columns per workgroup fill NTW tiles");
   constexpr int THREADS = 64 * NTW * KS;
@@ -754,14 +759,16 @@ __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) 
   const int64_t ws_base = (int64_t)((CW % 16 ? col : n0) / kBlock) * KB;
 
   // 1. first batch of this wave's weight loads (local k-blocks ks, ks+KS, ...)
-  u32x4 wl[kWideBatch][2];
-  float wsv[kWideBatch];
+  u32x4 wl[B][2];
+  float wsv[B];
   auto issue = [&](int b) {
 #pragma unroll
-    for (int j = 0; j < kWideBatch; ++j) {
+    for (int j = 0; j < B; ++j) {
       // unconditional: a k-block past the partition re-reads its last one
-      // (never multiplied), so the compiler can wait for each load alone
-      const int lk = min(ks + KS * (b * kWideBatch + j), kbp - 1);
+      // (never multiplied), so the compiler can wait for each load alone;
+      // with eight slots the re-reads would cost more than that wait
+      if (B == 8 && ks + KS * (b * B + j) >= kbp) continue;
+      const int lk = min(ks + KS * (b * B + j), kbp - 1);
       const int64_t ko = (int64_t)(kb0 + lk) * kBlock;
       wl[j][0] = *reinterpret_cast<const u32x4*>(wrow + ko);
       wl[j][1] = *reinterpret_cast<const u32x4*>(wrow + ko + 16);
@@ -785,14 +792,25 @@ __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) 
   issue(0);
   __builtin_amdgcn_sched_barrier(0);
 
-  // 2. stage the activation slab (rows past M are zero) and its scales
+  // 2. stage the activation slab and its scales (rows past M: zero scales)
   if constexpr (QX == 0) {
-    for (int c = tid; c < ROWS * kbp * 8; c += THREADS) {
-      const int row = c / (kbp * 8), rem = c % (kbp * 8), lk = rem >> 3, ch = rem & 7;
-      u32x4 v = {0u, 0u, 0u, 0u};
-      if (row < p.M)
-        v = *reinterpret_cast<const u32x4*>(p.a + (int64_t)row * p.K + (int64_t)(kb0 + lk) * kBlock + ch * 16);
-      *reinterpret_cast<u32x4*>(lds_a + (size_t)lk * ROWS * 128 + lds_off(row, ch)) = v;
+    if (reinterpret_cast<uintptr_t>(p.a) % 16 == 0) {
+      // eight rows of a k-block per DMA instruction, no registers between
+      // (rows past M repeat row M - 1: their products are never stored)
+      const int halves = (p.M + 7) / 8;
+      for (int c = wave; c < kbp * halves; c += NTW * KS) {
+        const int lk = c / halves, r0 = (c % halves) * 8, row = r0 + (lane >> 3);
+        const int ch = (lane & 7) ^ pipe::swizzle(row);
+        __builtin_amdgcn_global_load_lds(
+            (const void*)(p.a + (int64_t)min(row, p.M - 1) * p.K + (int64_t)(kb0 + lk) * kBlock + ch * 16),
+            (pipe::lds_void*)(lds_a + (size_t)lk * ROWS * 128 + r0 * 128), 16, 0, 0);
+      }
+    } else {
+      for (int c = tid; c < p.M * kbp * 8; c += THREADS) {
+        const int row = c / (kbp * 8), rem = c % (kbp * 8), lk = rem >> 3, ch = rem & 7;
+        *reinterpret_cast<u32x4*>(lds_a + (size_t)lk * ROWS * 128 + lds_off(row, ch)) =
+            *reinterpret_cast<const u32x4*>(p.a + (int64_t)row * p.K + (int64_t)(kb0 + lk) * kBlock + ch * 16);
+      }
     }
     for (int c = tid; c < ROWS * kbp; c += THREADS) {
       const int lk = c / ROWS, row = c % ROWS;
@@ -841,12 +859,12 @@ __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) 
   v4f acc[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
-  const int batches = (kbp + KS * kWideBatch - 1) / (KS * kWideBatch);
+  const int batches = (kbp + KS * B - 1) / (KS * B);
   for (int b = 0; b < batches; ++b) {
     if (b > 0) issue(b);
 #pragma unroll
-    for (int j = 0; j < kWideBatch; ++j) {
-      const int lk = ks + KS * (b * kWideBatch + j);
+    for (int j = 0; j < B; ++j) {
+      const int lk = ks + KS * (b * B + j);
       if (lk < kbp) {
         v8i bf;
         bf[0] = wl[j][0][0]; bf[1] = wl[j][0][1]; bf[2] = wl[j][0][2]; bf[3] = wl[j][0][3];
@@ -1088,11 +1106,11 @@ static void launch_small(const DenseArgs& a, int parts, hipStream_t s) {
 
 // Returns false (the caller takes another kernel) when the tile does not
 // fit or the kernel's dynamic LDS limit cannot be raised on this device.
-template <int MT, int NTW, int KS, int OUT, int SDT, int QX = 0, int CW = 16 * NTW>
+template <int MT, int NTW, int KS, int OUT, int SDT, int QX = 0, int CW = 16 * NTW, int B = 2>
 static bool launch_wide(const DenseArgs& a, int parts, hipStream_t s) {
   const size_t lds = wide_lds_bytes<MT, NTW, KS>(a.kb_per_part);
   if (lds > 160 * 1024 || a.N % CW) return false;
-  auto kern = dense_wide_kernel<MT, NTW, KS, OUT, SDT, QX, CW>;
+  auto kern = dense_wide_kernel<MT, NTW, KS, OUT, SDT, QX, CW, B>;
   // The 160 KB dynamic LDS limit, raised once per device for this kernel
   // (bit d: done on device d).
   static std::atomic<uint64_t> configured{0};
@@ -1125,15 +1143,27 @@ static int wide_columns(int n, int parts) {
   return 32;
 }
 
-// The M <= 16 wide kernel (MT = 1) at the column count wide_columns picks.
+// The M <= 16 wide kernel (MT = 1) at the column count wide_columns picks,
+// with B k-blocks in flight per wave.  (Fused, 24 columns, which fill the CUs
+// with 1024-thread workgroups, keep two: K=8192, N=6144, M=1 14.4 us, 14.7
+// with eight.)
+template <int OUT, int SDT, int QX, int B>
+static bool launch_wide_b(const DenseArgs& a, int parts, hipStream_t s) {
+  switch (wide_columns(a.N, parts)) {
+    case 24: return launch_wide<1, 2, 8, OUT, SDT, QX, 24, (QX != 0 ? 2 : B)>(a, parts, s);
+    case 16: return launch_wide<1, 1, 8, OUT, SDT, QX, 16, B>(a, parts, s);
+    case 8: return launch_wide<1, 1, 8, OUT, SDT, QX, 8, B>(a, parts, s);
+    default: return launch_wide<1, 2, 8, OUT, SDT, QX, 32, B>(a, parts, s);
+  }
+}
+
+// The same with B by depth.
 template <int OUT, int SDT, int QX = 0>
 static bool launch_wide_m16(const DenseArgs& a, int parts, hipStream_t s) {
-  switch (wide_columns(a.N, parts)) {
-    case 24: return launch_wide<1, 2, 8, OUT, SDT, QX, 24>(a, parts, s);
-    case 16: return launch_wide<1, 1, 8, OUT, SDT, QX, 16>(a, parts, s);
-    case 8: return launch_wide<1, 1, 8, OUT, SDT, QX, 8>(a, parts, s);
-    default: return launch_wide<1, 2, 8, OUT, SDT, QX>(a, parts, s);
-  }
+  if (a.kb_per_part <= 16) return launch_wide_b<OUT, SDT, QX, 2>(a, parts, s);
+  if constexpr (QX == 0)
+    if (a.kb_per_part <= 32) return launch_wide_b<OUT, SDT, QX, 4>(a, parts, s);
+  return launch_wide_b<OUT, SDT, QX, 8>(a, parts, s);
 }
 
 // Products of at most 64 rows and few k-blocks, while the direct small
@@ -1234,13 +1264,27 @@ int launch_dense(const DenseArgs& a, int parts, hipStream_t s) {
 // quantize + GEMM at M=1 / 4 / 16).  Larger batches use the split kernel.
 constexpr int kFusedQuantizeRows = 16;
 
+// Deeper than 16 k-blocks, every workgroup's own quantization of the slab
+// (rows * k-blocks groups, VALU-bound) passes the quantizer's launch: from
+// 192 groups while 16-column tiles come to at most one per CU, from 384 with
+// more columns, whose weights take longer.  fp8_linear, fused -> two launches
+// in us: K=8192, N=2048, M=16 23.0 -> 10.6, M=4 11.0 -> 9.4, M=2 8.7, 9.2;
+// K=N=4096, M=8 9.6 -> 8.6, M=4 7.3, 8.6; K=2560, N=4096, M=8 7.5, 7.9; K=6144,
+// N=8192, M=16 21.7 -> 16.6, M=4 13.2, 15.9.  The results are bit-identical.
+static bool quantize_apart(int64_t r, int64_t k, int64_t o) {
+  const int64_t kb = k / kBlock;
+  return kb > 16 && r * kb >= (o <= 16 * (int64_t)device_cus() ? 192 : 384);
+}
+
 template <int OUT, int SDT, int QX>
 static bool launch_fused_small_t(const DenseArgs& a, hipStream_t s) {
   // Every workgroup quantizes the whole slab, so above 8 rows the extra
   // workgroups of narrower tiles cost more than their smaller weight share
   // saves (M=16, N=6144: 7.26 us at 32 columns, 7.37 us at 24).
   if (a.M <= 8) return launch_wide_m16<OUT, SDT, QX>(a, 1, s);
-  if (a.M <= 16) return launch_wide<1, 2, 8, OUT, SDT, QX>(a, 1, s);
+  if (a.M <= 16)
+    return a.kb_per_part <= 16 ? launch_wide<1, 2, 8, OUT, SDT, QX>(a, 1, s)
+                               : launch_wide<1, 2, 8, OUT, SDT, QX, 32, 8>(a, 1, s);
   return false;
 }
 
@@ -1318,7 +1362,7 @@ static int check_linear(const void* x, int x_dtype, const uint8_t* w, const void
 static int run_fp8_linear(const void* x, int x_dtype, const uint8_t* w, const void* w_scales,
                           int scale_dtype, void* out, int out_dtype, void* workspace, int64_t r,
                           int64_t k, int64_t o, hipStream_t s) {
-  if (r <= kFusedQuantizeRows) {
+  if (r <= kFusedQuantizeRows && !quantize_apart(r, k, o)) {
     DenseArgs f{nullptr, nullptr, w, w_scales, out, o, 0, (int)r, (int)o, (int)k,
                 (int)(k / kBlock), scale_dtype, out_dtype, x, x_dtype};
     if (launch_fused_small(f, s))
