@@ -491,7 +491,7 @@ __global__ __launch_bounds__(dma::THREADS) void dense_dma_kernel(DenseArgs p) {
   // quarters of the last (partial) tiles that hold no row of A or of B
   plan.skip = (copies_a ? m0 : n0) + (wave & 3) * 64 >= (copies_a ? p.M : p.N);
 
-  const int a_row0 = (wave & 3) * 64, b_row0 = (wave >> 2) * 128;
+  const int a_row0 = dma::row_quarter(wave) * 64, b_row0 = (wave >> 2) * 128;
   const int col0 = n0 + b_row0;
   const bool live = m0 + a_row0 < p.M && col0 < p.N;  // wave-uniform
   // Weight scale of each k-block for this wave's 128-column block.  f32

@@ -851,8 +851,8 @@ __global__ __launch_bounds__(dma::THREADS) void expert_dma_kernel(ExpertArgs p) 
     plan.skip = false;
   }
 
-  const int wm = wave & 3, wn = wave >> 2;
-  const int a_row0 = wm * 64, b_row0 = wn * 128;
+  const int wn = wave >> 2;
+  const int a_row0 = dma::row_quarter(wave) * 64, b_row0 = wn * 128;
   // First output column of this wave; gate and up share its scale block.
   const int wcol = PAIRED ? n0 + b_row0 / 2 : n0 + b_row0;
   const float* w0 = dma::wtab[PAIRED ? 0 : wn];

@@ -1,7 +1,7 @@
 """Grouped expert products on the pipelined tiles (32 to 111 mean rows per
-expert): row tiles full, one over and one short, empty and one-row experts,
-k-block counts below and past the stages, packed rows, both scale dtypes,
-stores off alignment.  Bit for bit against the same call on a few rows at a
+expert) and the 256-row ones: row tiles full, one over and one short, empty
+and one-row experts, k-block counts below and past the stages, packed rows,
+both scale dtypes, stores off alignment.  Bit for bit against the same call on a few rows at a
 time, which runs on the decode tiles: every (row, column) is one float32
 chain in ascending k-block order on any tile, and so is the fused activation
 (src/akas/ops/moe/cuda.py:541-1354, :823-946)."""
@@ -33,6 +33,8 @@ def _routing(torch, sizes, top, dev):
     ([127, 128, 129, 2, 40, 60, 61, 93], 1024, 384),   # 80
     ([100, 101, 102, 103, 104, 105, 0, 121], 256, 128),  # 92
     ([192, 64, 1, 63, 66, 62, 32, 32], 1152, 640),     # 64
+    # 256-row tiles whose last one holds one to four quarters of rows
+    ([320, 321, 384, 385, 448, 449, 512, 513], 256, 384),  # 416
 ])
 @pytest.mark.parametrize("scale_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("packed", [False, True])

@@ -45,8 +45,8 @@ def _problem(dev, m, k, n, seed, scale_dtype="float32"):
     (300, 2048, 6144), (641, 1280, 2064), (999, 896, 2048), (770, 384, 1936),
     # 128x128 tiles, one workgroup per CU in two groups, and two per CU
     (513, 1408, 6000), (1290, 2048, 2000), (1100, 768, 5008), (2049, 1024, 2048),
-    # 256x256 tiles below a full round
-    (2049, 512, 6144),
+    # 256x256 tiles below a full round, one and three quarters of the last
+    (2049, 512, 6144), (2177, 384, 6144),
     # the largest depth, and the register-staged kernels past it
     (40, 16384, 272), (40, 16512, 272), (100, 16512, 256),
 ])
