@@ -130,10 +130,12 @@ struct GatherPlan {
   }
 };
 
-template <int S, class Plan>
+// NT: with the non-temporal hint (cache policy 2), for bytes that the launch
+// reads once.
+template <int S, bool NT, class Plan>
 AKAS_DEV void copy_piece(const Plan& p, int i, uint32_t ko) {
   __builtin_amdgcn_global_load_lds((const void*)p.ptr(i, ko),
-                                   (lds_void*)(stage_base<S>() + (p.blk0 + i) * 1024), 16, 0, 0);
+                                   (lds_void*)(stage_base<S>() + (p.blk0 + i) * 1024), 16, 0, NT ? 2 : 0);
 }
 template <int S, class Plan>
 AKAS_DEV void copy_scales(const Plan& p, int kb) {
@@ -141,11 +143,11 @@ AKAS_DEV void copy_scales(const Plan& p, int kb) {
     __builtin_amdgcn_global_load_lds((const void*)(p.as + (p.soff + kb)),
                                      (lds_void*)(stage_scales<S>() + (p.blk0 >> 3) * 64), 4, 0, 0);
 }
-template <int S, class Plan>
+template <int S, bool NT, class Plan>
 AKAS_DEV void copy_stage(const Plan& p, int kb) {
   const uint32_t ko = (uint32_t)kb * 128;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) copy_piece<S>(p, i, ko);
+  for (int i = 0; i < 8; ++i) copy_piece<S, NT>(p, i, ko);
   copy_scales<S>(p, kb);
 }
 
@@ -169,14 +171,14 @@ struct Acc {
 // waits for the MFMA results, and the other wave on the SIMD issues its
 // MFMAs meanwhile (keeping the previous products in flight instead costs 16
 // registers and measured no faster).
-template <int S, bool PAIRED, bool LIVE, class Plan>
+template <int S, bool PAIRED, bool LIVE, bool NT, class Plan>
 AKAS_DEV void multiply(const Plan& p, Acc& acc, int a_row0, int b_row0, float ws0, float ws1,
                        int lane, int kb_next) {
   const uint8_t* at = stage_base<S>();
   const uint8_t* bt = at + BM * 128;
   const uint32_t ko = (uint32_t)kb_next * 128;
   if constexpr (!LIVE) {
-    if (!p.skip) copy_stage<1 - S>(p, kb_next);
+    if (!p.skip) copy_stage<1 - S, NT>(p, kb_next);
     return;
   }
   v8i af[4];
@@ -190,7 +192,7 @@ AKAS_DEV void multiply(const Plan& p, Acc& acc, int a_row0, int b_row0, float ws
   }
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    copy_piece<1 - S>(p, j, ko);
+    copy_piece<1 - S, NT>(p, j, ko);
     if (j == 0) copy_scales<1 - S>(p, kb_next);
     const v8i bf = fragment(bt, b_row0 + 16 * j, lane);
     v4f cur[4];
@@ -213,20 +215,20 @@ AKAS_DEV void multiply(const Plan& p, Acc& acc, int a_row0, int b_row0, float ws
 // as a float2.  Every stage refills the other one with k-block
 // min(kb + 1, kb1 - 1): the refetch of the last block lands in a stage that
 // is never read again, and the closing barrier waits for it.
-template <bool PAIRED, bool LIVE, class Plan, class WS>
+template <bool PAIRED, bool LIVE, bool NT, class Plan, class WS>
 AKAS_DEV void run_(const Plan& p, Acc& acc, int a_row0, int b_row0, int kb0, int kb1, int lane, WS ws) {
-  if (LIVE || !p.skip) copy_stage<0>(p, kb0);
+  if (LIVE || !p.skip) copy_stage<0, NT>(p, kb0);
   float2 wcur = ws(kb0);
   __syncthreads();
   const int last = kb1 - 1;
   for (int kb = kb0; kb < kb1; kb += 2) {
     float2 wnext = ws(min(kb + 1, last));
-    multiply<0, PAIRED, LIVE>(p, acc, a_row0, b_row0, wcur.x, wcur.y, lane, min(kb + 1, last));
+    multiply<0, PAIRED, LIVE, NT>(p, acc, a_row0, b_row0, wcur.x, wcur.y, lane, min(kb + 1, last));
     __syncthreads();
     if (kb + 1 < kb1) {
       wcur = wnext;
       wnext = ws(min(kb + 2, last));
-      multiply<1, PAIRED, LIVE>(p, acc, a_row0, b_row0, wcur.x, wcur.y, lane, min(kb + 2, last));
+      multiply<1, PAIRED, LIVE, NT>(p, acc, a_row0, b_row0, wcur.x, wcur.y, lane, min(kb + 2, last));
       __syncthreads();
       wcur = wnext;
     }
@@ -234,11 +236,16 @@ AKAS_DEV void run_(const Plan& p, Acc& acc, int a_row0, int b_row0, int kb0, int
 }
 template <bool PAIRED, class Plan, class WS>
 AKAS_DEV void run(const Plan& p, Acc& acc, int a_row0, int b_row0, int kb0, int kb1, int lane, WS ws,
-                  bool live) {
-  if (live)  // wave-uniform: two loops, so the live one keeps its registers
-    run_<PAIRED, true>(p, acc, a_row0, b_row0, kb0, kb1, lane, ws);
+                  bool live, bool nt = false) {
+  // wave-uniform: loops of their own, so the live ones keep their registers
+  if (live && nt)
+    run_<PAIRED, true, true>(p, acc, a_row0, b_row0, kb0, kb1, lane, ws);
+  else if (live)
+    run_<PAIRED, true, false>(p, acc, a_row0, b_row0, kb0, kb1, lane, ws);
+  else if (nt)
+    run_<PAIRED, false, true>(p, acc, a_row0, b_row0, kb0, kb1, lane, ws);
   else
-    run_<PAIRED, false>(p, acc, a_row0, b_row0, kb0, kb1, lane, ws);
+    run_<PAIRED, false, false>(p, acc, a_row0, b_row0, kb0, kb1, lane, ws);
 }
 
 AKAS_DEV uint32_t pack2(float lo, float hi, int dt) {

@@ -68,6 +68,8 @@ struct ExpertArgs {
   int ws_dtype, prod_dtype, act_dtype;
   int max_tiles, tiles_n;
   int fair;  // progress-ordered wave priority in the k-loop (see expert_tiled_kernel)
+  // 256-row tiles: experts of one row tile take non-temporal weight loads
+  int stream;
 };
 
 // The work item of this workgroup: column block nb of row tile `tile` of
@@ -861,7 +863,9 @@ __global__ __launch_bounds__(dma::THREADS) void expert_dma_kernel(ExpertArgs p) 
   acc.clear();
   dma::run<PAIRED>(plan, acc, a_row0, b_row0, kb0, kb1, lane, [&](int kb) {
     return float2{w0[kb - kb0], PAIRED ? w1[kb - kb0] : 0.f};
-  }, row0 + a_row0 < count);  // a wave whose 64 rows are all padding only copies
+  },
+  row0 + a_row0 < count,  // a wave whose 64 rows are all padding only copies
+  wave >= 4 && p.stream && count <= BM);
 
   if constexpr (!PAIRED) {
     const int64_t rstride = (int64_t)p.parts * p.N;
@@ -1220,10 +1224,15 @@ static void launch_expert(ExpertArgs a, hipStream_t s) {
         <<<grid, 64 * WMW * WNW, 0, s>>>(a);
 }
 
+// Whether a launch's weights come to at least 96 MB, more than a call can
+// leave of them in the 256 MB last-level cache for the next.
+static bool weights_past_cache(const ExpertArgs& a, int64_t bytes_per_expert) {
+  return std::min<int64_t>(a.E, (int64_t)a.r * a.top) * bytes_per_expert >= (96ll << 20);
+}
+
 // Whether a decode launch loads its weights with the non-temporal hint: when
-// it streams at least 96 MB of them, more than a call can leave in the 256 MB
-// last-level cache for the next, and most experts have one row tile, so that
-// no second tile reads them again.  Without the hint every line streamed
+// they are past the last-level cache and most experts have one row tile, so
+// that no second tile reads them again.  Without the hint every line streamed
 // displaces another from the caches on its way (64 experts, 2048 -> 1536 ->
 // 2048, whole block: 256 tokens 131.3 -> 122.4 us, 64 125.6 -> 116.1, 400
 // 166.4 -> 158.9; 256 experts of 512 and a shared one, 64 tokens 157.8 ->
@@ -1231,8 +1240,7 @@ static void launch_expert(ExpertArgs a, hipStream_t s) {
 // and with weights that stay in the cache from call to call (32 experts, 1024
 // -> 512, 64 tokens: 31.6 -> 35.0).
 static bool stream_weights(const ExpertArgs& a, int64_t bytes_per_expert) {
-  const int64_t routes = (int64_t)a.r * a.top;
-  return std::min<int64_t>(a.E, routes) * bytes_per_expert >= (96ll << 20) && routes / a.E <= 28;
+  return weights_past_cache(a, bytes_per_expert) && (int64_t)a.r * a.top / a.E <= 28;
 }
 
 // A decode launch with or without the hint (the modes that decode runs).
@@ -1263,6 +1271,13 @@ template <int MODE, int OUT>
 static void launch_expert_dma(ExpertArgs a, hipStream_t s) {
   a.max_tiles = (int)capacity_tiles(a.r, a.top, a.E, dma::BM);
   a.tiles_n = paired_mode(MODE) ? a.N / (dma::BN / 2) : a.N / dma::BN;
+  // Experts whose rows fit one tile have their weights read once by this
+  // launch: with the hint those lines displace no others, neither the larger
+  // experts' weights nor the activations (64 experts of 1536, skewed routing,
+  // whole block: 3000 tokens 324.5 -> 316.2 us, 6000 460.9 -> 439.6).  On the
+  // pipelined tiles it gained 2-4% with uniform routing and lost 1-2% with
+  // skewed, so those keep the plain copies.
+  a.stream = weights_past_cache(a, (int64_t)a.N * a.K * (paired_mode(MODE) ? 2 : 1));
   dim3 grid((unsigned)(a.max_tiles * a.tiles_n), (unsigned)a.parts);
   expert_dma_kernel<MODE, OUT><<<grid, dma::THREADS, 0, s>>>(a);
 }
