@@ -6,6 +6,7 @@
 // selection compares IEEE float32 scores with lowest-index tie breaking and
 // the route compaction is an ordered block scan, never an atomic cursor.
 #include "common.h"
+#include "device_info.h"
 #include "moe_launch.h"
 #include "quant_group.h"
 
@@ -353,13 +354,13 @@ __global__ __launch_bounds__(256) void decode_router_quantize_kernel(
 //
 // The flattened entries g = row * top + rank of ids are already in route
 // order, so an expert's route at position q is its q-th matching entry.
-// Workgroup (c, e) owns chunk c (`passes` times 1024 * V entries) for expert
+// Workgroup (e, c) owns chunk c (`passes` times 1024 * V entries) for expert
 // e: it counts the matches in every earlier chunk itself (16-byte loads that
 // wait for nothing), then numbers its own chunk's by a block scan per pass.
-// One workgroup per expert walking all entries was a serial chain of load,
-// scan and barrier per 1024 rows: 34.4 us at 16384 rows x 4 over 64 experts,
-// now 12.0; 6.9 -> 5.1 us at 1500 rows.  V = 16 and at most kRouteChunks
-// chunks keep the entries that are counted again in proportion to all.
+// Experts and chunks both spread the work, and only chunks count entries
+// again, so there are as many chunks as leave one workgroup per CU
+// (launch_routes): with up to 16 chunks whatever the experts, 40000 rows x 4
+// took 69 us over 64 experts (4 chunks: 18.4) and 220 over 512 (1 chunk: 59).
 //
 // A route names the entry row * ld + rank (ld = top for quantized_routes).
 // With ld = top + 1, one more expert (index `experts`) routes every row at
@@ -369,69 +370,93 @@ __global__ __launch_bounds__(256) void decode_router_quantize_kernel(
 // ---------------------------------------------------------------------------
 constexpr int kRouteChunks = 16;
 
-template <int V, bool VEC>
+// ACT: 0 every row is active; 1 a flag per entry, loaded beside the ids (an
+// activity load behind each match would wait for the ids first); 2 top is a
+// multiple of four, so four aligned entries share one row and one flag.
+template <int V, bool VEC, int ACT>
 __global__ __launch_bounds__(1024) void routes_kernel(const int32_t* __restrict__ ids,
                                                       const int32_t* __restrict__ active,
                                                       int32_t* __restrict__ counts,
                                                       int32_t* __restrict__ routes, int64_t rows,
                                                       int top, int ld, int experts, int passes) {
   static_assert(V % 4 == 0 && V <= 32, "entries per thread: whole 16-byte loads, one mask");
-  __shared__ int2 wave_tot[16];  // matches of a wave: before the chunk, in the pass
-  const int e = blockIdx.y;
+  __shared__ int wave_earlier[16], wave_tot[2][16];  // matches of a wave: before the chunk, in a pass
+  const int e = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // rows * top is below 2^31, the last chunk's end below 2^32
   const uint32_t n = (uint32_t)(rows * top), chunk = 1024u * V * passes;
-  const uint32_t c0 = blockIdx.x * chunk;
+  const uint32_t c0 = blockIdx.y * chunk;
   int32_t* out = routes + (int64_t)e * rows;
   if (e == experts) {  // the shared expert: row order, rank top
-    for (int64_t row = (int64_t)blockIdx.x * 1024 + tid; row < rows; row += (int64_t)gridDim.x * 1024)
+    for (int64_t row = (int64_t)blockIdx.y * 1024 + tid; row < rows; row += (int64_t)gridDim.y * 1024)
       out[row] = (int32_t)(row * ld + top);
-    if (blockIdx.x == 0 && tid == 0) counts[e] = (int32_t)rows;
+    if (blockIdx.y == 0 && tid == 0) counts[e] = (int32_t)rows;
     return;
   }
-  // Matches among entries g .. g+3 (bit i: entry g+i), none past the end.
-  auto match4 = [&](uint32_t g) -> uint32_t {
-    int v[4];
-    if (VEC && g + 4 <= n) {
-      const int4 q = *reinterpret_cast<const int4*>(ids + g);
-      v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+  // Matches among the N entries from g on (bit i: entry g+i), none past the
+  // end.  Every load is independent: ids and flags in one round trip.
+  auto match = [&](uint32_t g, auto N) -> uint32_t {
+    constexpr int kN = decltype(N)::value;
+    uint32_t m = 0, row = 0, rank = 0;
+    if constexpr (ACT != 0) row = g / (uint32_t)top, rank = g - row * (uint32_t)top;
+    int v[kN], a[kN];
+    if (VEC && g + kN <= n) {
+#pragma unroll
+      for (int i = 0; i < kN; i += 4) {
+        const int4 q = *reinterpret_cast<const int4*>(ids + g + i);
+        v[i] = q.x; v[i + 1] = q.y; v[i + 2] = q.z; v[i + 3] = q.w;
+      }
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = g + i < n ? ids[g + i] : -1;
+      for (int i = 0; i < kN; ++i) v[i] = g + i < n ? ids[g + i] : -1;
     }
-    uint32_t m = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) m |= (uint32_t)(v[i] == e) << i;
-    if (active && m) {
+    for (int i = 0; i < kN; i += ACT == 2 ? 4 : 1) {
+      if constexpr (ACT == 0) break;
+      a[i] = active[min(row, (uint32_t)rows - 1)];
+      rank += ACT == 2 ? 4 : 1;
+      if (rank == (uint32_t)top) rank = 0, ++row;
+    }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (((m >> i) & 1u) && active[(g + i) / top] == 0) m &= ~(1u << i);
+    for (int i = 0; i < kN; i += 4) {
+      uint32_t q = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool hit = ACT == 1 ? (v[i + j] == e) & (a[i + j] != 0) : v[i + j] == e;
+        q |= (uint32_t)hit << (i + j);
+      }
+      m |= ACT == 2 && a[i] == 0 ? 0u : q;
     }
     return m;
   };
-  int earlier = 0;
-#pragma unroll 4
-  for (uint32_t g = 4 * tid; g < c0; g += 4096) earlier += __builtin_popcount(match4(g));
-  earlier = wave_sum_i(earlier);
   int64_t base = 0;  // matches before the pass
+  if (c0 > 0) {
+    int earlier = 0;
+#pragma unroll 4
+    for (uint32_t g = 4 * tid; g < c0; g += 4096) earlier += __builtin_popcount(match(g, DtypeTag<4>{}));
+    earlier = wave_sum_i(earlier);
+    if (lane == 0) wave_earlier[wave] = earlier;  // read after the first pass's barrier
+  }
   for (int p = 0; p < passes; ++p) {
     const uint32_t g0 = c0 + (uint32_t)p * (1024 * V) + tid * V;
-    uint32_t mask = 0;
-#pragma unroll
-    for (int i = 0; i < V; i += 4)
-      if (g0 + i < n) mask |= match4(g0 + i) << i;
+    const uint32_t mask = g0 < n ? match(g0, DtypeTag<V>{}) : 0;
     const int cnt = __builtin_popcount(mask);
     const int incl = wave_inclusive_scan(cnt, lane);
-    if (p > 0) __syncthreads();  // the last pass's totals are read
-    if (lane == 63) wave_tot[wave] = make_int2(p == 0 ? earlier : 0, incl);
+    // two sets of totals in turn: the barrier of the pass between says that
+    // every wave has read the set written here
+    int* tot = wave_tot[p & 1];
+    if (lane == 63) tot[wave] = incl;
     __syncthreads();
+    if (p == 0 && c0 > 0) {
+#pragma unroll
+      for (int w = 0; w < 16; ++w) base += wave_earlier[w];
+    }
     int before = 0, total = 0;
 #pragma unroll
     for (int w = 0; w < 16; ++w) {
-      const int2 t = wave_tot[w];
-      base += t.x;
-      before += w < wave ? t.y : 0;
-      total += t.y;
+      const int t = tot[w];
+      before += w < wave ? t : 0;
+      total += t;
     }
     // Positions past the row length (only reachable with duplicate ids in
     // one row, which top-k selection never produces) are dropped.
@@ -442,32 +467,128 @@ __global__ __launch_bounds__(1024) void routes_kernel(const int32_t* __restrict_
     }
     base += total;
   }
-  if (blockIdx.x == gridDim.x - 1) {  // the last chunk knows the count
+  if (blockIdx.y == gridDim.y - 1) {  // the last chunk knows the count
     const int64_t used = base < rows ? base : rows;
     for (int64_t i = used + tid; i < rows; i += 1024) out[i] = -1;
     if (tid == 0) counts[e] = (int32_t)used;
   }
 }
 
-// V = 4 spreads up to 16384 entries over up to four chunks per expert; more
-// entries take V = 16.
+// V (entries per thread and pass) and chunks, by what was fastest over 1 to
+// 40000 rows, 8 to 1024 experts and 1 to 16 ranks: four entries at one rank
+// or few entries, sixteen where four share a row's flag; as many chunks as
+// keep about one workgroup per CU.  In us, one workgroup per expert walking
+// 1024 rows a pass -> this: 16384 x 8 over 64 experts 77.1 -> 14.7, over 256
+// 81.5 -> 21.1; 2000 x 8 over 256 11.7 -> 4.7; 4097 x 4 over 64 11.6 -> 5.2;
+// 1 x 4 3.24 -> 3.03.
 static void launch_routes(const int32_t* ids, const int32_t* active, int32_t* counts,
                           int32_t* routes, int64_t r, int experts, int top, int ld,
                           hipStream_t s) {
   const int64_t n = r * top;
   const bool vec = reinterpret_cast<uintptr_t>(ids) % 16 == 0;
-  auto go = [&](auto V, auto VEC) {
+  int64_t most = kRouteChunks;
+  while (most > 1 && most * experts > device_cus()) most /= 2;
+  auto go = [&](auto V, auto VEC, auto ACT) {
     constexpr int v = decltype(V)::value;
     const int64_t blocks = n > 0 ? (n + 1024 * v - 1) / (1024 * v) : 1;
-    const int64_t passes = (blocks + kRouteChunks - 1) / kRouteChunks;
-    dim3 grid((unsigned)((blocks + passes - 1) / passes), (unsigned)(experts + (ld > top)));
-    routes_kernel<v, decltype(VEC)::value != 0><<<grid, 1024, 0, s>>>(
+    const int64_t passes = (blocks + most - 1) / most;
+    dim3 grid((unsigned)(experts + (ld > top)), (unsigned)((blocks + passes - 1) / passes));
+    routes_kernel<v, decltype(VEC)::value != 0, decltype(ACT)::value><<<grid, 1024, 0, s>>>(
         ids, active, counts, routes, r, top, ld, experts, (int)passes);
   };
-  if (n <= 16384)
-    vec ? go(DtypeTag<4>{}, DtypeTag<1>{}) : go(DtypeTag<4>{}, DtypeTag<0>{});
-  else
-    vec ? go(DtypeTag<16>{}, DtypeTag<1>{}) : go(DtypeTag<16>{}, DtypeTag<0>{});
+  auto by_flags = [&](auto VEC) {
+    if (active && top % 4 != 0) {
+      if (top == 1 || n <= 4096)
+        go(DtypeTag<4>{}, VEC, DtypeTag<1>{});
+      else
+        go(DtypeTag<8>{}, VEC, DtypeTag<1>{});
+    } else if (n <= 8192) {
+      active ? go(DtypeTag<8>{}, VEC, DtypeTag<2>{}) : go(DtypeTag<8>{}, VEC, DtypeTag<0>{});
+    } else {
+      active ? go(DtypeTag<16>{}, VEC, DtypeTag<2>{}) : go(DtypeTag<16>{}, VEC, DtypeTag<0>{});
+    }
+  };
+  vec ? by_flags(DtypeTag<1>{}) : by_flags(DtypeTag<0>{});
+}
+
+// top = 4 with flags: four consecutive rows per thread (one 16-byte load of
+// their ids each, one of their activity flags), 4096 rows per pass, and the
+// next pass's loads in flight while this pass is scanned and written: one
+// workgroup per expert.  Taken where that leaves no CU idle, or where one pass
+// is all there is (routes4_fits); elsewhere chunks win.
+__global__ __launch_bounds__(1024) void routes4_kernel(const int32_t* __restrict__ ids,
+                                                       const int32_t* __restrict__ active,
+                                                       int32_t* __restrict__ counts,
+                                                       int32_t* __restrict__ routes, int64_t rows) {
+  constexpr int RPT = 4, PASS = 1024 * RPT;
+  __shared__ int wave_tot[16];
+  const int e = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int32_t* out = routes + (int64_t)e * rows;
+  // rows past the end read row 0 (their flags are masked below)
+  auto load = [&](int64_t r0, int4 (&id)[RPT], int4& act) {
+    const int64_t row = r0 + (int64_t)tid * RPT;
+    const int64_t safe = row + RPT <= rows ? row : 0;
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) id[i] = reinterpret_cast<const int4*>(ids)[safe + i];
+    act = *reinterpret_cast<const int4*>(active + safe);
+  };
+  int4 id[RPT], act, nid[RPT], nact;
+  load(0, id, act);
+  int64_t base = 0;
+  for (int64_t r0 = 0; r0 < rows; r0 += PASS) {
+    if (r0 + PASS < rows) load(r0 + PASS, nid, nact);
+    const int64_t row = r0 + (int64_t)tid * RPT;
+    const int a[RPT] = {act.x, act.y, act.z, act.w};
+    uint32_t mask[RPT];
+    int cnt = 0;
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      const bool live = row + i < rows && a[i] != 0;
+      const int4 v = id[i];
+      mask[i] = live ? (uint32_t)(v.x == e) | ((uint32_t)(v.y == e) << 1) |
+                           ((uint32_t)(v.z == e) << 2) | ((uint32_t)(v.w == e) << 3)
+                     : 0u;
+      cnt += __builtin_popcount(mask[i]);
+    }
+    const int incl = wave_inclusive_scan(cnt, lane);
+    if (lane == 63) wave_tot[wave] = incl;
+    __syncthreads();
+    int before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const int t = wave_tot[w];
+      before += w < wave ? t : 0;
+      total += t;
+    }
+    int64_t pos = base + before + incl - cnt;
+#pragma unroll
+    for (int i = 0; i < RPT; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if ((mask[i] >> k) & 1u) {
+          if (pos < rows) out[pos] = (int32_t)((row + i) * 4 + k);
+          ++pos;
+        }
+    base += total;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) id[i] = nid[i];
+    act = nact;
+  }
+  const int64_t used = base < rows ? base : rows;
+  for (int64_t i = used + tid; i < rows; i += 1024) out[i] = -1;
+  if (tid == 0) counts[e] = (int32_t)used;
+}
+
+// Above 2500 rows (below, the other kernel's lighter passes win: 2000 rows
+// over 64 experts 4.23 us, 3.80), with more experts than CUs (512 experts,
+// 16384 rows: 22.8 us, 26.6 on the other kernel) or a single pass (4000 rows:
+// 4.86, 4.99).
+static bool routes4_fits(const int32_t* ids, const int32_t* active, int64_t r, int experts,
+                         int top) {
+  return top == 4 && active && r % 4 == 0 && r > 2500 && (experts > device_cus() || r <= 4096) &&
+         reinterpret_cast<uintptr_t>(active) % 16 == 0 && reinterpret_cast<uintptr_t>(ids) % 16 == 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -857,7 +978,10 @@ int launch_decode_router_quantize(const float* logits, int32_t* ids, float* weig
 
 void launch_quantized_routes(const int32_t* ids, const int32_t* active, int32_t* counts,
                              int32_t* routes, int64_t r, int experts, int top, hipStream_t s) {
-  launch_routes(ids, active, counts, routes, r, experts, top, top, s);
+  if (routes4_fits(ids, active, r, experts, top))
+    routes4_kernel<<<experts, 1024, 0, s>>>(ids, active, counts, routes, r);
+  else
+    launch_routes(ids, active, counts, routes, r, experts, top, top, s);
 }
 
 void launch_routes_with_shared(const int32_t* ids, int32_t* counts, int32_t* routes, int64_t r,
