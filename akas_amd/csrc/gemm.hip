@@ -734,8 +734,8 @@ constexpr size_t wide_lds_bytes(int kbp) {
 // B: k-blocks of weights in flight per wave.  Two cover a 2048-deep product
 // (16 k-blocks over KS = 8 waves); deeper ones take four or eight: in batches
 // of two, each batch waited a memory round trip for its own loads (fp8_linear
-// M=1, K=8192, N=2048 9.2 -> 8.2 us; at K=2048 eight slots lose, N=6144 5.3 ->
-// 6.1).
+// M=1, K=8192, N=2048 9.2 -> 8.2 us, with bf16 scales 9.6 -> 8.1; at K=2048
+// eight slots lose, N=6144 5.3 -> 6.1).
 template <int MT, int NTW, int KS, int OUT, int SDT, int QX = 0, int CW = 16 * NTW, int B = 2>
 __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) {
   static_assert(CW > 16 * (NTW - 1) && CW <= 16 * NTW, "columns per workgroup fill NTW tiles");
@@ -759,8 +759,20 @@ __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) 
   const int64_t ws_base = (int64_t)((CW % 16 ? col : n0) / kBlock) * KB;
 
   // 1. first batch of this wave's weight loads (local k-blocks ks, ks+KS, ...)
+  // bf16 scales have no scalar load, and converting one beside its load waits
+  // for it and for every weight load before it, a memory round trip per slot.
+  // So lane l loads that of the wave's l-th k-block once, ahead of the
+  // weights, and each use converts its own (fp8_linear, eight slots, M=1, us:
+  // K=N=4096 8.0 -> 6.4; K=4096, N=12288 18.7 -> 14.5; two slots 7.0, 15.6).
+  // At most 77 k-blocks fit the slab, ten per wave.
+  constexpr bool LANE_SCALES = SDT == AKAS_DTYPE_BF16 && CW % 16 == 0;
+  uint32_t wlane = 0;
+  if constexpr (LANE_SCALES) {
+    wlane = reinterpret_cast<const uint16_t*>(p.ws)[ws_base + kb0 + min(ks + KS * lane, kbp - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+  }
   u32x4 wl[B][2];
-  float wsv[B];
+  uint32_t wsv[B];
   auto issue = [&](int b) {
 #pragma unroll
     for (int j = 0; j < B; ++j) {
@@ -772,7 +784,11 @@ __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) 
       const int64_t ko = (int64_t)(kb0 + lk) * kBlock;
       wl[j][0] = *reinterpret_cast<const u32x4*>(wrow + ko);
       wl[j][1] = *reinterpret_cast<const u32x4*>(wrow + ko + 16);
-      wsv[j] = load_scale_t<SDT>(p.ws, ws_base + kb0 + lk);
+      const int64_t at = ws_base + kb0 + lk;
+      if constexpr (SDT == AKAS_DTYPE_F32)
+        wsv[j] = reinterpret_cast<const uint32_t*>(p.ws)[at];
+      else if constexpr (!LANE_SCALES)
+        wsv[j] = reinterpret_cast<const uint16_t*>(p.ws)[at];
     }
   };
   // Fused quantize: the first pass of activation loads goes out before the
@@ -870,15 +886,17 @@ __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) 
         bf[0] = wl[j][0][0]; bf[1] = wl[j][0][1]; bf[2] = wl[j][0][2]; bf[3] = wl[j][0][3];
         bf[4] = wl[j][1][0]; bf[5] = wl[j][1][1]; bf[6] = wl[j][1][2]; bf[7] = wl[j][1][3];
         const uint8_t* at = lds_a + (size_t)lk * ROWS * 128;
+        const uint32_t raw = LANE_SCALES ? __builtin_amdgcn_readlane(wlane, b * B + j) : wsv[j];
+        const float ws = __uint_as_float(SDT == AKAS_DTYPE_F32 ? raw : raw << 16);
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
           const v8i af = lds_fragment(at, 16 * i, lane);
           const float4 s4 = *reinterpret_cast<const float4*>(lds_s + lk * ROWS + 16 * i + 4 * g);
           const v4f pr = mfma_e4m3(af, bf);
-          acc[i][0] = __builtin_fmaf(pr[0], s4.x * wsv[j], acc[i][0]);
-          acc[i][1] = __builtin_fmaf(pr[1], s4.y * wsv[j], acc[i][1]);
-          acc[i][2] = __builtin_fmaf(pr[2], s4.z * wsv[j], acc[i][2]);
-          acc[i][3] = __builtin_fmaf(pr[3], s4.w * wsv[j], acc[i][3]);
+          acc[i][0] = __builtin_fmaf(pr[0], s4.x * ws, acc[i][0]);
+          acc[i][1] = __builtin_fmaf(pr[1], s4.y * ws, acc[i][1]);
+          acc[i][2] = __builtin_fmaf(pr[2], s4.z * ws, acc[i][2]);
+          acc[i][3] = __builtin_fmaf(pr[3], s4.w * ws, acc[i][3]);
         }
       }
     }

@@ -16,7 +16,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("m,k,n", [
     (1, 2176, 512), (2, 2560, 6144), (3, 8192, 2048), (16, 2304, 6144), (15, 2560, 4096),
     (9, 4096, 1040), (8, 4224, 2048), (7, 8064, 272), (16, 8192, 528), (5, 8192, 6144),
-    (16, 8832, 256), (16, 9216, 256), (4, 4096, 24 * 16)])
+    (16, 8832, 256), (16, 9216, 256), (4, 4096, 24 * 16),
+    # 32 columns, fused: eight slots filled in part, full and over
+    (1, 2176, 8192), (9, 2304, 7680), (5, 9728, 8192)])
 @pytest.mark.parametrize("scale_dtype", ["float32", "bfloat16"])
 def test_deep_rows(dev, m, k, n, scale_dtype):
     import torch
