@@ -1170,7 +1170,17 @@ static bool launch_wide_b(const DenseArgs& a, int parts, hipStream_t s) {
   switch (wide_columns(a.N, parts)) {
     case 24: return launch_wide<1, 2, 8, OUT, SDT, QX, 24, (QX != 0 ? 2 : B)>(a, parts, s);
     case 16: return launch_wide<1, 1, 8, OUT, SDT, QX, 16, B>(a, parts, s);
-    case 8: return launch_wide<1, 1, 8, OUT, SDT, QX, 8, B>(a, parts, s);
+    case 8:
+      // Fused, eight slots take 132 registers: one workgroup per CU.  Where a
+      // grid has more and their slabs would share a CU, fewer slots let them:
+      // four while one batch holds the depth (K=4096, N=3072, M=1: 7.1 us,
+      // two slots 7.5, eight 8.6), else two (K=4224: 8.2, four 8.6, eight 9.1).
+      if constexpr (QX != 0 && B == 8)
+        if ((int64_t)(a.N / 8) * parts > device_cus() &&
+            2 * wide_lds_bytes<1, 1, 8>(a.kb_per_part) <= 160 * 1024)
+          return a.kb_per_part <= 32 ? launch_wide<1, 1, 8, OUT, SDT, QX, 8, 4>(a, parts, s)
+                                     : launch_wide<1, 1, 8, OUT, SDT, QX, 8, 2>(a, parts, s);
+      return launch_wide<1, 1, 8, OUT, SDT, QX, 8, B>(a, parts, s);
     default: return launch_wide<1, 2, 8, OUT, SDT, QX, 32, B>(a, parts, s);
   }
 }

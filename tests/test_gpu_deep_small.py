@@ -18,7 +18,9 @@ pytestmark = pytest.mark.gpu
     (9, 4096, 1040), (8, 4224, 2048), (7, 8064, 272), (16, 8192, 528), (5, 8192, 6144),
     (16, 8832, 256), (16, 9216, 256), (4, 4096, 24 * 16),
     # 32 columns, fused: eight slots filled in part, full and over
-    (1, 2176, 8192), (9, 2304, 7680), (5, 9728, 8192)])
+    (1, 2176, 8192), (9, 2304, 7680), (5, 9728, 8192),
+    # 8 columns, more workgroups than CUs: four slots and two, and on codes quantized apart
+    (1, 2176, 3072), (3, 4224, 2320), (12, 2176, 3072), (16, 2304, 3072)])
 @pytest.mark.parametrize("scale_dtype", ["float32", "bfloat16"])
 def test_deep_rows(dev, m, k, n, scale_dtype):
     import torch
