@@ -1299,9 +1299,16 @@ constexpr int kFusedQuantizeRows = 16;
 // in us: K=8192, N=2048, M=16 23.0 -> 10.6, M=4 11.0 -> 9.4, M=2 8.7, 9.2;
 // K=N=4096, M=8 9.6 -> 8.6, M=4 7.3, 8.6; K=2560, N=4096, M=8 7.5, 7.9; K=6144,
 // N=8192, M=16 21.7 -> 16.6, M=4 13.2, 15.9.  The results are bit-identical.
+// Above eight rows, where the fused form has 32 columns per workgroup, and
+// the product alone would run more workgroups than CUs, 96 groups more
+// (N=3072: K=2176, M=12 7.1, 7.9; K=3072, M=12 8.8, 8.4; N=5888, K=6144, M=9
+// 15.1, 16.0).
 static bool quantize_apart(int64_t r, int64_t k, int64_t o) {
-  const int64_t kb = k / kBlock;
-  return kb > 16 && r * kb >= (o <= 16 * (int64_t)device_cus() ? 192 : 384);
+  const int64_t kb = k / kBlock, cus = device_cus();
+  int64_t least = o <= 16 * cus ? 192 : 384;
+  if (r > 8 && o % 32 == 0 && wide_columns((int)o, 1) < 32 && o / wide_columns((int)o, 1) > cus)
+    least += 96;
+  return kb > 16 && r * kb >= least;
 }
 
 template <int OUT, int SDT, int QX>
