@@ -407,10 +407,17 @@ AKAS_DEV float swiglu_elem(float g, float u) {
 // half the instruction's bytes and no scale register to issue with it,
 // against the scaled form with unit scales (127), which gives the same bits
 // (256x256 prefill tiles, M=8192: 1,984 -> 2,022 TFLOP/s at K=2048, N=6144;
-// 2,000 -> 2,045 at N=8192; M=2048: 1,858 -> 1,912).
+// 2,000 -> 2,045 at N=8192; M=2048: 1,858 -> 1,912).  SCALED takes that form:
+// the register-staged dense tiles are scheduled worse around the plain one
+// (128x128 tiles, K=17408, N=2048: M=300 132.6 us, plain 149.8; M=1000 135.7,
+// 154.7), every other kernel is as fast or faster with it.
+template <bool SCALED = false>
 AKAS_DEV v4f mfma_e4m3(const v8i& a, const v8i& b) {
   v4f z = {0.f, 0.f, 0.f, 0.f};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, z, 0, 0, 0, 0, 0, 0);
+  if constexpr (SCALED)
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, z, 0, 0, 0, 127, 0, 127);
+  else
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, z, 0, 0, 0, 0, 0, 0);
 }
 
 // ---------------------------------------------------------------------------

@@ -127,8 +127,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void dense_tiled_kernel(Den
     const int k = kb + (J);                                                          \
     const int cur = (k - kb0) & 1;                                                   \
     if (k < kb1)                                                                     \
-      mma_stage<MT, NT>(acc, lds + cur * STAGE, lds + cur * STAGE + BM * 128,        \
-                        lds_as[cur], a_row0, b_row0, ws_cur, lane);                  \
+      mma_stage<MT, NT, false, true>(acc, lds + cur * STAGE, lds + cur * STAGE + BM * 128, \
+                                     lds_as[cur], a_row0, b_row0, ws_cur, lane);     \
     constexpr int ns = ((J) + 1) % DEPTH;                                            \
     plan.stash(lds + (cur ^ 1) * STAGE, ring_a[ns], ring_b[ns]);                     \
     if (tid < BM) lds_as[cur ^ 1][tid] = ras[ns];                                    \

@@ -117,8 +117,8 @@ AKAS_DEV v8i lds_fragment(const uint8_t* tile, int row0, int lane) {
 //   interleaved 16 rows at a time).
 // acc += P * (as[m] * ws) with one fresh MFMA product P per 16x16 tile.  The
 // scale FMAs of n-tile j-1 are issued while the MFMAs of n-tile j run, so MT
-// independent products are always in flight.
-template <int MT, int NT, bool PAIRED = false>
+// independent products are always in flight.  SCALED: see mfma_e4m3.
+template <int MT, int NT, bool PAIRED = false, bool SCALED = false>
 AKAS_DEV void mma_stage(Acc<MT, NT>& acc, const uint8_t* a_tile, const uint8_t* b_tile,
                         const float* as_stage, int a_row0, int b_row0, float ws0, int lane,
                         float ws1 = 0.f) {
@@ -139,7 +139,7 @@ AKAS_DEV void mma_stage(Acc<MT, NT>& acc, const uint8_t* a_tile, const uint8_t* 
     const v8i bf = lds_fragment(b_tile, b_row0 + 16 * j, lane);
     v4f cur[MT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) cur[i] = mfma_e4m3(af[i], bf);
+    for (int i = 0; i < MT; ++i) cur[i] = mfma_e4m3<SCALED>(af[i], bf);
     if (j > 0) {
 #pragma unroll
       for (int i = 0; i < MT; ++i)
