@@ -43,9 +43,9 @@ AKAS_DEV void grouped_tile(int id, int tiles_m, int tiles_n, int G, int& tm, int
 //
 // DEPTH k-blocks are in flight per workgroup in a register ring in front of
 // the two LDS stages: at k-block kb the ring holds kb+1 .. kb+DEPTH, so the
-// HBM latency of a load is covered by DEPTH k-block multiplies.  Decode-sized
-// launches (few tiles, 16 k-blocks) need DEPTH 3-4; prefill tiles fill the
-// GPU with enough workgroups that DEPTH 1 suffices.
+// HBM latency of a load is covered by DEPTH k-block multiplies.  Two for the
+// small tiles of few rows; larger tiles have enough workgroups that one
+// suffices.
 // ---------------------------------------------------------------------------
 template <int BM, int BN, int WAVES_M, int WAVES_N, int DEPTH, int OUT, int SDT>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void dense_tiled_kernel(DenseArgs p) {
@@ -142,13 +142,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void dense_tiled_kernel(Den
   for (int kb = kb0; kb < kb1; kb += DEPTH) {
     AKAS_RING_STEP(0)
     AKAS_RING_STEP(1)
-    AKAS_RING_STEP(2)
-    AKAS_RING_STEP(3)
-    AKAS_RING_STEP(4)
-    AKAS_RING_STEP(5)
   }
 #undef AKAS_RING_STEP
-  static_assert(DEPTH >= 1 && DEPTH <= 6, "prefetch depth 1..6");
+  static_assert(DEPTH == 1 || DEPTH == 2, "ring steps above");
 
   const int64_t obase = (int64_t)part * p.part_stride;
 #pragma unroll
@@ -700,7 +696,7 @@ __global__ __launch_bounds__(256) void dense_small_kernel(DenseArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// Wide small-M MFMA GEMM (M <= 32): one workgroup of NTW x KS waves covers
+// Wide small-M MFMA GEMM (M <= 64): one workgroup of NTW x KS waves covers
 // 16*NTW columns and the partition's whole k range.  The activation slab
 // (codes and scales of all its rows) is staged in LDS once per workgroup,
 // every wave issues all of its weight loads up front (k-blocks strided by
@@ -1202,38 +1198,27 @@ static bool shallow_rows(const DenseArgs& a) {
   return a.M <= 64 && a.kb_per_part <= (a.M <= 32 ? 12 : 4) && a.N <= 16 * device_cus();
 }
 
-// Kernel choice by shape, in order:
-//   M <= 16                                   the wide kernel (activations
-//                                             staged once per workgroup in LDS)
-//   16 < M <= 256 with 2048-deep partitions   the split kernel, where estimated
-//                                             faster than the engine below
-//   16 < M <= 64, few k-blocks                the direct small kernel (shallow_rows)
-//   16 < M <= 32, 9 to 16 k-blocks, columns   the wide kernel (K=1536, N=6144,
-//     past one 16-column tile per CU          M=24: 6.6 us, 7.0 pipelined)
-//   otherwise                                 the pipelined engine or the 256x256
-//                                             DMA kernel, the tile estimated fastest
-// Codes off 16-byte alignment and partitions past kPipeMaxKb k-blocks take
-// the register-staged kernels: 128x128 tiles where N is a multiple of 128,
-// else (and up to 64 rows) the direct small kernel in 64-row slices.
+// The register-staged kernels, by rows: the wide kernel where its slab fits,
+// else the direct small kernel; 64x64 tiles to 256 rows, then 256x128 tiles
+// where they come to two per CU, else 128x128 (us, 64x64 against 128x128 or,
+// at N=2112, 64-row slices of the small kernel: K=17408, M=200, N=2048 93.6,
+// 151.9; N=2112 93.7, 218).  Tiles need N to be a multiple of their columns;
+// other shapes take 64-row slices of the small kernel.  Up to eight k-blocks
+// of 17 to 32 rows the small kernel is the faster one (K=640, N=6144, M=20:
+// 4.8 us, the wide kernel 6.0).
 template <int OUT, int SDT>
-static void launch_dense_t(const DenseArgs& a, int parts, hipStream_t s) {
-  if (a.M <= 16 && launch_wide_m16<OUT, SDT>(a, parts, s)) return;
-  if (split_applies(a, parts)) {
-    launch_split_m<0, OUT, SDT>(a, parts, s);
-    return;
-  }
-  if (a.M <= 32 && a.kb_per_part > 8 && a.kb_per_part <= 16 && a.N > 16 * device_cus() &&
-      launch_wide<2, 2, 8, OUT, SDT>(a, parts, s))
-    return;
-  if (a.M > 16 && pipe_fits(a) && !shallow_rows(a)) {
-    switch (dense_tile(a, parts)) {
-      case kTile64x64: launch_pipe<Pipe64x64, OUT, SDT>(a, parts, s); break;
-      case kTile64x128: launch_pipe<Pipe64x128, OUT, SDT>(a, parts, s); break;
-      case kTile128x128: launch_pipe<Pipe128x128, OUT, SDT>(a, parts, s); break;
-      case kTile128x128x2: launch_pipe<Pipe128x128x2, OUT, SDT>(a, parts, s); break;
-      default: launch_dma<OUT, SDT>(a, parts, s);
-    }
-  } else if (a.M > 64 && a.N % 128 == 0) {
+static void launch_staged(const DenseArgs& a, int parts, hipStream_t s) {
+  if (a.M <= 64) {
+    if (a.M > 16 && !shallow_rows(a) && (a.M > 32 || a.kb_per_part > 8) &&
+        (a.M <= 32 ? launch_wide<2, 2, 8, OUT, SDT>(a, parts, s)
+                   : launch_wide<4, 2, 8, OUT, SDT>(a, parts, s)))
+      return;
+    launch_small<OUT, SDT>(a, parts, s);
+  } else if (a.M <= 256 && a.N % 64 == 0) {
+    launch_tiled<64, 64, 2, 2, 2, OUT, SDT>(a, parts, s);
+  } else if (a.N % 128 == 0 && (int64_t)((a.M + 255) / 256) * (a.N / 128) >= 512) {
+    launch_tiled<256, 128, 4, 2, 1, OUT, SDT>(a, parts, s);
+  } else if (a.N % 128 == 0) {
     launch_tiled<128, 128, 2, 2, 1, OUT, SDT>(a, parts, s);
   } else {
     const int esz = OUT == AKAS_DTYPE_F32 ? 4 : 2;
@@ -1245,6 +1230,45 @@ static void launch_dense_t(const DenseArgs& a, int parts, hipStream_t s) {
       b.out = reinterpret_cast<char*>(a.out) + (int64_t)m0 * a.ldo * esz;
       launch_small<OUT, SDT>(b, parts, s);
     }
+  }
+}
+
+// Kernel choice by shape, in order:
+//   M <= 16                                   the wide kernel (activations
+//                                             staged once per workgroup in LDS)
+//   16 < M <= 256 with 2048-deep partitions   the split kernel, where estimated
+//                                             faster than the engine below
+//   16 < M <= 64, few k-blocks                the direct small kernel (shallow_rows)
+//   16 < M <= 32, 9 to 16 k-blocks, columns   the wide kernel (K=1536, N=6144,
+//     past one 16-column tile per CU          M=24: 6.6 us, 7.0 pipelined)
+//   otherwise                                 the pipelined engine or the 256x256
+//                                             DMA kernel, the tile estimated fastest
+// Codes off 16-byte alignment and partitions past kPipeMaxKb k-blocks take
+// the register-staged kernels (launch_staged).
+template <int OUT, int SDT>
+static void launch_dense_t(const DenseArgs& a, int parts, hipStream_t s) {
+  if (a.M <= 16 && launch_wide_m16<OUT, SDT>(a, parts, s)) return;
+  if (split_applies(a, parts)) {
+    launch_split_m<0, OUT, SDT>(a, parts, s);
+    return;
+  }
+  if (!pipe_fits(a)) {
+    launch_staged<OUT, SDT>(a, parts, s);
+    return;
+  }
+  if (a.M <= 32 && a.kb_per_part > 8 && a.kb_per_part <= 16 && a.N > 16 * device_cus() &&
+      launch_wide<2, 2, 8, OUT, SDT>(a, parts, s))
+    return;
+  if (a.M <= 16 || shallow_rows(a)) {
+    launch_small<OUT, SDT>(a, parts, s);
+    return;
+  }
+  switch (dense_tile(a, parts)) {
+    case kTile64x64: launch_pipe<Pipe64x64, OUT, SDT>(a, parts, s); break;
+    case kTile64x128: launch_pipe<Pipe64x128, OUT, SDT>(a, parts, s); break;
+    case kTile128x128: launch_pipe<Pipe128x128, OUT, SDT>(a, parts, s); break;
+    case kTile128x128x2: launch_pipe<Pipe128x128x2, OUT, SDT>(a, parts, s); break;
+    default: launch_dma<OUT, SDT>(a, parts, s);
   }
 }
 

@@ -28,3 +28,23 @@ def dev():
 
     _lib.load()  # fails loudly when the extension is missing
     return torch.device("cuda:0")
+
+
+@pytest.fixture
+def launched(dev):
+    """``launched(call)``: names of this library's kernels that ``call()``
+    launches, in order, template arguments included."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+
+    def names(call):
+        torch.cuda.synchronize()
+        with profile(activities=[ProfilerActivity.CUDA]) as p:
+            call()
+            torch.cuda.synchronize()
+        # "void akas::kernel<...>(akas::Args)"
+        found = [e.name.split("akas::", 1)[1].rsplit("(", 1)[0] for e in p.events()
+                 if "akas::" in e.name and "(" in e.name]
+        return [name.replace("akas::", "") for name in found]
+
+    return names

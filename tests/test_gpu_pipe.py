@@ -48,7 +48,8 @@ def _problem(dev, m, k, n, seed, scale_dtype="float32"):
     # 256x256 tiles below a full round, one and three quarters of the last
     (2049, 512, 6144), (2177, 384, 6144),
     # the largest depth, and the register-staged kernels past it
-    (40, 16384, 272), (40, 16512, 272), (100, 16512, 256),
+    (40, 16384, 272), (40, 16512, 272), (100, 16512, 256), (130, 16512, 192),
+    (300, 16512, 272),
 ])
 @pytest.mark.parametrize("scale_dtype", ["float32", "bfloat16"])
 def test_mid_size_linear(dev, m, k, n, scale_dtype):
@@ -87,7 +88,8 @@ def test_mid_size_partitions(dev, m, k, n, parts):
 
 
 @pytest.mark.parametrize("out_dtype", ["float32", "bfloat16", "float16"])
-@pytest.mark.parametrize("m,n", [(300, 1040), (130, 512)])
+@pytest.mark.parametrize("m,n", [(300, 1040), (130, 512), (17, 512), (50, 544), (65, 576),
+                                 (300, 384), (4097, 4096)])
 def test_mid_size_unaligned_operands(dev, m, n, out_dtype):
     """An output off 16-byte alignment takes element stores, codes off it the
     register-staged kernels; neither writes outside its rows."""
