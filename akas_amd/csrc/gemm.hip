@@ -319,13 +319,13 @@ __global__ __launch_bounds__(64 * kSplitQuarters * MH) void dense_split_kernel(D
   const int wl_row0 = mh * (BN / MH);
   const uint8_t* wsrc = p.w + (int64_t)(n0 + wl_row0 + wl_row) * p.K + (int64_t)kb0 * kBlock + 16 * wl_chunk;
   u32x4 wl[WLOADS];
-  // Non-temporal: a decode step reads each weight once, from HBM (24 linears
-  // over 302 MB of weights in one graph, M=40 240 -> 224.5 us, M=128 283 ->
-  // 271; weights that fit the last-level cache, M=64 98.4 -> 99.4).
+  // (No non-temporal hint: a launch cannot know whether a decode step's weights
+  // stay in the last-level cache from step to step.  24 linears over 302 MB,
+  // M=40: 240 us, 224.5 with it; but 8192 x 2048 at M=64 from the cache 8.5,
+  // 9.9.)
   auto issue_w = [&]() {
 #pragma unroll
-    for (int q = 0; q < WLOADS; ++q)
-      wl[q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wsrc + (int64_t)(2 * q) * p.K));
+    for (int q = 0; q < WLOADS; ++q) wl[q] = *reinterpret_cast<const u32x4*>(wsrc + (int64_t)(2 * q) * p.K);
   };
   if constexpr (AFIRST) {
     issue_a();
