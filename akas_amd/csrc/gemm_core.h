@@ -35,8 +35,8 @@ AKAS_DEV int lds_off(int row, int chunk) { return row * 128 + ((chunk ^ ((row & 
 // the loads use scalar-base addressing with one VGPR per address.  Rows past the end of an operand are clamped to a valid row
 // by the caller: their products land in rows/columns that are never stored
 // or carry a zero scale, so no branch is needed in the copy loop.
-// STREAM: B (the weights) is loaded with the non-temporal hint, for weights
-// that this launch reads once and from HBM.
+// STREAM: B (the weights) is loaded with the non-temporal hint where `nt`
+// (uniform) says so, for weights that this launch reads once and from HBM.
 template <int BM, int BN, int THREADS, bool STREAM = false>
 struct StagePlan {
   static constexpr int RSTEP = THREADS / 8;
@@ -55,6 +55,7 @@ struct StagePlan {
   uint32_t b_step;        // bytes between this thread's successive B rows
   int dst0;               // LDS offset of this thread's first chunk
   bool a_live = true;     // this thread moves A chunks (always unless A_PART)
+  bool nt = false;
 
   // Staging registers are kept in two small arrays (A chunks, B chunks):
   // one 128-byte array of uint4 is past what the alloca promotion keeps in
@@ -67,10 +68,18 @@ struct StagePlan {
   }
   AKAS_DEV void fetch_b(int kb, u32x4 (&rb)[CB]) const {
     const uint32_t ko = (uint32_t)kb * kBlock;
+    if (STREAM && nt) {
+      // (the empty asm keeps the branches' loads from being merged, which
+      // drops the hint)
+      asm volatile("");
 #pragma unroll
-    for (int j = 0; j < CB; ++j) {
-      const u32x4* src = reinterpret_cast<const u32x4*>(b_base + (b_off + j * b_step + ko));
-      rb[j] = STREAM ? __builtin_nontemporal_load(src) : *src;
+      for (int j = 0; j < CB; ++j)
+        rb[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(b_base + (b_off + j * b_step + ko)));
+      asm volatile("");
+    } else {
+#pragma unroll
+      for (int j = 0; j < CB; ++j)
+        rb[j] = *reinterpret_cast<const u32x4*>(b_base + (b_off + j * b_step + ko));
     }
   }
   AKAS_DEV void fetch(int kb, u32x4 (&ra)[CA], u32x4 (&rb)[CB]) const {

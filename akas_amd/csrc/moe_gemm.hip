@@ -68,7 +68,8 @@ struct ExpertArgs {
   int ws_dtype, prod_dtype, act_dtype;
   int max_tiles, tiles_n;
   int fair;  // progress-ordered wave priority in the k-loop (see expert_tiled_kernel)
-  // 256-row tiles: experts of one row tile take non-temporal weight loads
+  // Live experts from which weights read by one row tile take non-temporal
+  // loads (see hint_experts; the 256-row tiles and the STREAM kernels)
   int stream;
 };
 
@@ -78,8 +79,9 @@ struct ExpertArgs {
 // fastest, before the XCD remap: the grid is sized for the most tiles the
 // routes can produce, and a remap over the whole grid left the dead tail --
 // up to a quarter of the grid -- on the last XCDs, idling them.
+// live: experts with rows.
 struct Item {
-  int nb, expert, tile, count;
+  int nb, expert, tile, count, live;
 };
 
 // Position of logical tile t among the row tiles n (one expert per lane) of
@@ -112,6 +114,7 @@ AKAS_DEV bool find_item_64(int c, int r, int bm, int tiles_n, int lane, Item& it
   const int id = xcd_remap(blockIdx.x, items);
   if (id >= items) return false;
   it.nb = id % tiles_n;
+  it.live = __builtin_popcountll(__ballot(c > 0));
   int base = 0;
   return tile_in_chunk(n, c, 0, id / tiles_n, r, lane, base, it);
 }
@@ -121,10 +124,12 @@ AKAS_DEV bool find_item(const int32_t* counts, int experts, int r, int bm, int t
   if (experts <= 64)
     return find_item_64(lane < experts ? max(counts[lane], 0) : 0, r, bm, tiles_n, lane, it);
   int total = 0;
+  it.live = 0;
   for (int e0 = 0; e0 < experts; e0 += 64) {
     const int e = e0 + lane;
     const int c = e < experts ? max(counts[e], 0) : 0;
     total += wave_sum_i((c + bm - 1) / bm);
+    it.live += __builtin_popcountll(__ballot(c > 0));
   }
   const int items = total * tiles_n;
   const int id = xcd_remap(blockIdx.x, items);
@@ -248,9 +253,12 @@ AKAS_DEV bool find_item_hist(const int* hist, int experts, int r, int bm, int ti
   if (experts <= 64)
     return find_item_64(lane < experts ? min(hist[lane], r) : 0, r, bm, tiles_n, lane, it);
   int total = 0;
+  it.live = 0;
   for (int e0 = 0; e0 < experts; e0 += 64) {
     const int e = e0 + lane;
-    total += wave_sum_i(e < experts ? (min(hist[e], r) + bm - 1) / bm : 0);
+    const int c = e < experts ? min(hist[e], r) : 0;
+    total += wave_sum_i((c + bm - 1) / bm);
+    it.live += __builtin_popcountll(__ballot(c > 0));
   }
   const int items = total * tiles_n;
   const int id = xcd_remap(blockIdx.x, items);
@@ -468,7 +476,8 @@ AKAS_DEV void wave_priority_by_progress(int done, int total) {
 // SIMD, so that three workgroups share a CU.
 // SCAN: the workgroup scans ids itself (scan_entries) instead of reading the
 // route tables, and writes them for the launches after it.
-// STREAM: the weights take non-temporal loads (see stream_weights).
+// STREAM: where p.stream experts are live (see hint_experts), those of one row
+// tile take non-temporal weight loads.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int MODE, int OUT, int SDT, int STAGES = 0,
           int SCAN = 0, bool STREAM = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N)
@@ -556,6 +565,7 @@ void expert_tiled_kernel(ExpertArgs p) {
       plan.b_step = (uint32_t)Plan::RSTEP * (uint32_t)p.K;
     }
     plan.dst0 = lds_off(row, ch);
+    if constexpr (STREAM) plan.nt = __builtin_amdgcn_readfirstlane(item.live) >= p.stream && count <= BM;
   }
   // Gathered source rows and scatter destinations of this tile.  The first
   // weight k-block is requested before they are known: after the route
@@ -865,7 +875,7 @@ __global__ __launch_bounds__(dma::THREADS) void expert_dma_kernel(ExpertArgs p) 
     return float2{w0[kb - kb0], PAIRED ? w1[kb - kb0] : 0.f};
   },
   row0 + a_row0 < count,  // a wave whose 64 rows are all padding only copies
-  wave >= 4 && p.stream && count <= BM);
+  wave >= 4 && item.live >= p.stream && count <= BM);
 
   if constexpr (!PAIRED) {
     const int64_t rstride = (int64_t)p.parts * p.N;
@@ -1224,31 +1234,36 @@ static void launch_expert(ExpertArgs a, hipStream_t s) {
         <<<grid, 64 * WMW * WNW, 0, s>>>(a);
 }
 
-// Whether a launch's weights come to at least 96 MB, more than a call can
-// leave of them in the 256 MB last-level cache for the next.
-static bool weights_past_cache(const ExpertArgs& a, int64_t bytes_per_expert) {
-  return std::min<int64_t>(a.E, (int64_t)a.r * a.top) * bytes_per_expert >= (96ll << 20);
+// Live experts whose weights come to 272 MB, more than the 256 MB last-level
+// cache holds: with so many a launch finds none of its weights there whatever
+// ran before, and loads them with the non-temporal hint, so that the lines it
+// streams displace no others (the down projection's weights, of an earlier
+// layer or of the last call).  With fewer, weights that would have stayed from
+// call to call are lost.  Whole blocks called again and again, us, no hint ->
+// hint: 64 experts of 1536, 256 tokens 128.1 -> 111.2, 64 123.4 -> 107.9; 48
+// experts, 64 tokens 103 -> 90; below the line, 48 experts of 768 on 1536 (162
+// MB a block), 256 tokens 50.7 -> 58.8, and 129 experts of 512 (258 MB of gate
+// and up), 400 tokens 95.0 -> 99.3.  The line holds for the live experts,
+// which only the device knows: under skewed routing 64 tokens reach so few of
+// 64 experts that the hint costs 65.2 -> 70.
+static int hint_experts(int64_t bytes_per_expert) {
+  return (int)std::min<int64_t>(((272ll << 20) + bytes_per_expert - 1) / bytes_per_expert, 0x7FFFFFFF);
 }
 
-// Whether a decode launch loads its weights with the non-temporal hint: when
-// they are past the last-level cache and most experts have one row tile, so
-// that no second tile reads them again.  Without the hint every line streamed
-// displaces another from the caches on its way (64 experts, 2048 -> 1536 ->
-// 2048, whole block: 256 tokens 131.3 -> 122.4 us, 64 125.6 -> 116.1, 400
-// 166.4 -> 158.9; 256 experts of 512 and a shared one, 64 tokens 157.8 ->
-// 152.5).  With two row tiles per expert it loses (640 tokens 160.4 -> 180.7),
-// and with weights that stay in the cache from call to call (32 experts, 1024
-// -> 512, 64 tokens: 31.6 -> 35.0).
-static bool stream_weights(const ExpertArgs& a, int64_t bytes_per_expert) {
-  return weights_past_cache(a, bytes_per_expert) && (int64_t)a.r * a.top / a.E <= 28;
+// Whether a decode launch can reach that many, with most experts in one row
+// tile, so that no second tile reads their weights again (two tiles per
+// expert: 640 tokens 160.4 -> 180.7).
+static bool stream_weights(const ExpertArgs& a) {
+  const int64_t mean = (int64_t)a.r * a.top / a.E;
+  return std::min<int64_t>(a.E, (int64_t)a.r * a.top) >= a.stream && mean <= 28;
 }
 
 // A decode launch with or without the hint (the modes that decode runs).
 template <int BM, int BN, int MODE, int OUT, int STAGES = 0, int SCAN = 0>
-static void launch_decode_expert(const ExpertArgs& a, hipStream_t s) {
+static void launch_decode_expert(ExpertArgs a, hipStream_t s) {
   if constexpr (MODE == kPartial || MODE == kSwigluFp8) {
-    const int64_t bytes = (int64_t)a.N * a.K * (paired_mode(MODE) ? 2 : 1);
-    if (stream_weights(a, bytes)) {
+    a.stream = hint_experts((int64_t)a.N * a.K * (paired_mode(MODE) ? 2 : 1));
+    if (stream_weights(a)) {
       launch_expert<BM, BN, 1, 4, MODE, OUT, STAGES, SCAN, true>(a, s);
       return;
     }
@@ -1274,10 +1289,10 @@ static void launch_expert_dma(ExpertArgs a, hipStream_t s) {
   // Experts whose rows fit one tile have their weights read once by this
   // launch: with the hint those lines displace no others, neither the larger
   // experts' weights nor the activations (64 experts of 1536, skewed routing,
-  // whole block: 3000 tokens 324.5 -> 316.2 us, 6000 460.9 -> 439.6).  On the
+  // whole block: 3000 tokens 324 -> 307 us, 5000 426 -> 411).  On the
   // pipelined tiles it gained 2-4% with uniform routing and lost 1-2% with
   // skewed, so those keep the plain copies.
-  a.stream = weights_past_cache(a, (int64_t)a.N * a.K * (paired_mode(MODE) ? 2 : 1));
+  a.stream = hint_experts((int64_t)a.N * a.K * (paired_mode(MODE) ? 2 : 1));
   dim3 grid((unsigned)(a.max_tiles * a.tiles_n), (unsigned)a.parts);
   expert_dma_kernel<MODE, OUT><<<grid, dma::THREADS, 0, s>>>(a);
 }

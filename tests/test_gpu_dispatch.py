@@ -45,3 +45,44 @@ def _linear(dev, m, k, n, *, quantized=False, offset=0):
 def test_staged_kernels(dev, launched, m, k, n, offset, kernel):
     names = launched(_linear(dev, m, k, n, quantized=True, offset=offset))
     assert names and all(name.startswith(kernel) for name in names), names
+
+
+def _experts(dev, t, h, f, experts, top, *, offset=0):
+    """The gate/up and down products of a routed batch, as calls without
+    arguments; codes start ``offset`` bytes off 16-byte alignment."""
+    import torch
+    from akas_amd import ops
+
+    def codes(*shape):
+        n = int(torch.Size(shape).numel())
+        return torch.ones(n + offset, dtype=torch.uint8, device=dev)[offset:].view(shape)
+
+    def scales(*shape):
+        return torch.ones(shape, dtype=torch.float32, device=dev)
+
+    ids = (torch.arange(t * top, device=dev, dtype=torch.int32) % experts).view(t, top)
+    counts, routes = ops.quantized_routes(ids, torch.ones(t, dtype=torch.int32, device=dev),
+                                          experts=experts)
+    up, us = codes(experts, f, h), scales(experts, f // 128, h // 128)
+    down, ds = codes(experts, h, f), scales(experts, h // 128, f // 128)
+    x, xs = codes(t, h), scales(t, h // 128)
+    act, acs = codes(t, top, f), scales(t, top, f // 128)
+    kw = dict(r=t, top=top)
+    return (lambda: ops.fp8_expert_swiglu(x, xs, up, us, up, us, counts, routes, **kw),
+            lambda: ops.expert_partial(act, acs, down, ds, counts, routes, routed_input=True, **kw))
+
+
+# Decode kernels that may take the non-temporal hint end in "true": only where
+# the launch's weights can pass the last-level cache.
+@pytest.mark.parametrize("t,h,f,experts,top,up,down", [
+    (256, 2048, 1536, 64, 4, True, False),  # 403 and 201 MB
+    (16, 2048, 1536, 64, 4, True, False),
+    (10, 2048, 1536, 64, 4, False, False),  # 40 routes reach at most 252 MB
+    (256, 1536, 768, 48, 2, False, False),  # 113 and 57 MB
+    (400, 2048, 512, 129, 4, False, False),  # 258 MB
+])
+def test_hint_needs_more_than_the_cache(dev, launched, t, h, f, experts, top, up, down):
+    for call, hint in zip(_experts(dev, t, h, f, experts, top), (up, down)):
+        names = launched(call)
+        assert len(names) == 1 and names[0].startswith("expert_tiled_kernel<"), names
+        assert names[0].endswith("true>" if hint else "false>"), names
