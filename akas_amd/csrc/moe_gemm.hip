@@ -1312,6 +1312,18 @@ static bool expert_pipe_fits(const ExpertArgs& a) {
          aligned(a.xw) && aligned(a.xw2);
 }
 
+// Whether the 256-row tiles of a batch (column_blocks of them per row tile)
+// are too few for the CUs.
+static bool few_tiles(const ExpertArgs& a, int64_t mean, int64_t column_blocks) {
+  return (int64_t)a.E * ((mean + 255) / 256) * column_blocks < (int64_t)device_cus() * 3 / 4;
+}
+
+// Mean rows of a routed expert: a shared expert outside the bank, which takes
+// every row, is not one of them.
+static int64_t routed_mean(const ExpertArgs& a) {
+  return a.xw ? (int64_t)a.r * (a.top - 1) / (a.E - 1) : (int64_t)a.r * a.top / a.E;
+}
+
 // Row tile by the mean rows per expert (the down projection of 64 experts,
 // 1536 -> 2048, us):
 //   below 32     32-row tiles (mean 16: 40; 25: 41.4, 35.6 on the next)
@@ -1320,14 +1332,23 @@ static bool expert_pipe_fits(const ExpertArgs& a) {
 //                33.5, but mean 25: 29.9, 31.5 on 64 rows)
 //   to 111       128-row pipelined tiles, two per CU (mean 94: 47.7 -> 44.9)
 //   beyond       DMA-fed 256-row tiles (mean 125: 53.0 against 58.1; 94: 51.4
-//                against 44.9)
+//                against 44.9); from 128 where they are few (32 experts,
+//                512 -> 1024, mean 114: 18.2, 15.4 on 128 rows) or the output
+//                is f32 (the same, 22.1, 18.7; 64 experts, 768 -> 1536, 43.6,
+//                39.8)
+// Where one 64-row tile per expert just fills the CUs, the second tiles of a
+// few experts take a round of their own, and 32-row tiles stay to a mean of 48
+// (64 experts, 768 -> 1536, mean 47: 24.1, 25.7; mean 40: 23.6, 21.5).
 // expert_combine, and codes off the pipelined engine's alignment, keep
 // 32-row tiles to a mean of 48 and register-staged 128-row tiles after.
 template <int OUT, int MODE = kPartial>
 static void launch_partial(const ExpertArgs& a, hipStream_t s) {
-  const int64_t mean = (int64_t)a.r * a.top / a.E;
-  const bool piped = MODE == kPartial && mean >= 32 && expert_pipe_fits(a);
-  if (mean >= 112 && expert_dma_fits(a, dma::BN)) {
+  const int64_t mean = (int64_t)a.r * a.top / a.E, slots = 3 * (int64_t)device_cus();
+  const int64_t tiles64 = (int64_t)a.E * (a.N / 128) * a.parts;
+  const bool full = mean > 40 && mean <= 48 && tiles64 <= slots && tiles64 * 9 / 8 > slots;
+  const bool piped = MODE == kPartial && mean >= 32 && !full && expert_pipe_fits(a);
+  const bool late = piped && (OUT == AKAS_DTYPE_F32 || few_tiles(a, mean, a.N / 256 * a.parts));
+  if (routed_mean(a) >= (late ? 128 : 112) && expert_dma_fits(a, dma::BN)) {
     launch_expert_dma<MODE, OUT>(a, s);
     return;
   }
@@ -1379,15 +1400,21 @@ static void launch_paired(const ExpertArgs& a, hipStream_t s) {
   } else if constexpr (!SCAN) {
     // Above 48 mean rows: the DMA-fed 256-row tiles from a mean of 100 (64
     // experts, 2048 -> 1536: mean 106 121.6 us against 132.0 on 128 rows; 94:
-    // 121 against 104.3), unless too few of them for the CUs and one or two
-    // 128-row tiles hold an expert (32 experts, 1024 -> 512, mean 175: 26.7,
-    // 24.5; 275: 28.7, 39.7).  Before, the pipelined 128-row tile, or its
-    // 64-row one while 128-row tiles would leave CUs idle (the same 32
-    // experts, mean 62: 22.0 register-staged, 18.9 on 128 rows, 15.3 on 64).
+    // 121 against 104.3), f32 gate and up partials from 120 (mean 104 139.9,
+    // 133.8; 64 experts, 1536 -> 768, mean 114 61.3, 59.5; 125 63.0, 76.4).
+    // Too few of them for the CUs, 128-row tiles to a mean of 127 (32 experts,
+    // 1024 -> 512, mean 114: f32 partials 29.9, 26.9), on the pipelined engine
+    // to 240 while any routing leaves them in one round (mean 128; at 187,
+    // skewed, the block took 57.7 us, 63.6; 8 experts to 240).  Before, the
+    // pipelined 128-row tile, or its 64-row one while 128-row tiles would
+    // leave CUs idle (the same 32 experts, mean 62: 22.0 register-staged, 18.9
+    // on 128 rows, 15.3 on 64).
     const int64_t column_blocks = a.N / 128 * a.parts;
-    const bool few = (int64_t)a.E * ((mean + 255) / 256) * column_blocks < cus * 3 / 4;
+    const bool few = few_tiles(a, mean, column_blocks);
     const bool piped = MODE == kSwigluFp8 && expert_pipe_fits(a);
-    if (aligned && mean >= 100 && !(piped && few && mean <= 240) && expert_dma_fits(a, dma::BN / 2)) {
+    const bool one_round = ((int64_t)a.r * a.top / 128 + a.E) * column_blocks <= cus;
+    const int64_t least = few ? (piped && one_round ? 241 : 128) : MODE == kPairPartial ? 120 : 100;
+    if (aligned && routed_mean(a) >= least && expert_dma_fits(a, dma::BN / 2)) {
       launch_expert_dma<MODE, OUT>(a, s);
       return;
     }

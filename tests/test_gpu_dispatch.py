@@ -69,7 +69,8 @@ def _experts(dev, t, h, f, experts, top, *, offset=0):
     act, acs = codes(t, top, f), scales(t, top, f // 128)
     kw = dict(r=t, top=top)
     return (lambda: ops.fp8_expert_swiglu(x, xs, up, us, up, us, counts, routes, **kw),
-            lambda: ops.expert_partial(act, acs, down, ds, counts, routes, routed_input=True, **kw))
+            lambda **kv: ops.expert_partial(act, acs, down, ds, counts, routes, routed_input=True,
+                                            **kw, **kv))
 
 
 # Decode kernels that may take the non-temporal hint end in "true": only where
@@ -86,3 +87,71 @@ def test_hint_needs_more_than_the_cache(dev, launched, t, h, f, experts, top, up
         names = launched(call)
         assert len(names) == 1 and names[0].startswith("expert_tiled_kernel<"), names
         assert names[0].endswith("true>" if hint else "false>"), names
+
+
+# Row tiles of the expert products at the means where the choice turns.
+@pytest.mark.parametrize("mean,h,f,experts,up,down,down_f32", [
+    (104, 512, 2048, 64, "dma", "pipe", "pipe"),
+    (114, 2048, 1536, 64, "dma", "dma", "pipe"),
+    (128, 2048, 512, 64, "dma", "dma", "dma"),
+    (120, 1024, 512, 32, "pipe", "pipe", "pipe"),  # few 256-row tiles
+    (128, 1024, 512, 32, "pipe", "dma", "dma"),  # one round however they fall
+    (187, 1024, 512, 32, "dma", "dma", "dma"),
+    (240, 1024, 512, 8, "pipe", "dma", "dma"),
+    (242, 1024, 512, 8, "dma", "dma", "dma"),
+    (40, 1536, 768, 64, "tiled", "pipe", "pipe"),
+    (47, 1536, 768, 64, "tiled", "tiled", "tiled"),  # 768 tiles of 64 rows fill the CUs
+    (49, 1536, 768, 64, "pipe", "pipe", "pipe"),
+])
+def test_expert_row_tiles(dev, launched, mean, h, f, experts, up, down, down_f32):
+    import torch
+
+    gate_up, product = _experts(dev, mean * experts // 4, h, f, experts, 4)
+    half = lambda: product(output_dtype=torch.bfloat16)  # noqa: E731
+    for call, kernel in ((gate_up, up), (half, down), (product, down_f32)):
+        names = launched(call)
+        assert len(names) == 1 and names[0].startswith(f"expert_{kernel}_kernel<"), names
+
+
+@pytest.mark.parametrize("mean,f,experts,kernel", [
+    (104, 1536, 64, "tiled"), (119, 768, 64, "tiled"), (120, 768, 64, "dma"),
+    (127, 512, 32, "tiled"), (128, 512, 32, "dma")])
+def test_pair_partial_row_tiles(dev, launched, mean, f, experts, kernel):
+    import torch
+    from akas_amd import ops
+
+    t, h, top = mean * experts // 4, 1024, 4
+    ids = (torch.arange(t * top, device=dev, dtype=torch.int32) % experts).view(t, top)
+    counts, routes = ops.quantized_routes(ids, torch.ones(t, dtype=torch.int32, device=dev),
+                                          experts=experts)
+    w = torch.ones((experts, f, h), dtype=torch.uint8, device=dev)
+    s = torch.ones((experts, f // 128, h // 128), dtype=torch.float32, device=dev)
+    x = torch.ones((t, h), dtype=torch.uint8, device=dev)
+    xs = torch.ones((t, h // 128), dtype=torch.float32, device=dev)
+    names = launched(lambda: ops.expert_pair_partial(x, xs, w, s, w, s, counts, routes, r=t, top=top))
+    assert len(names) == 1 and names[0].startswith(f"expert_{kernel}_kernel<"), names
+
+
+@pytest.mark.parametrize("t,kernel", [(1599, "pipe"), (1600, "dma")])
+def test_shared_block_row_tiles(dev, launched, t, kernel):
+    """The mean that chooses the gate/up tiles is that of the routed experts
+    (100 at 1600 rows x 4 over 64), without the shared one's rows."""
+    import torch
+    from akas_amd import moe
+
+    experts, h, f = 64, 1024, 512
+
+    def weights(*lead):
+        def one(n, k):
+            return (torch.ones((*lead, n, k), dtype=torch.uint8, device=dev),
+                    torch.ones((*lead, n // 128, k // 128), dtype=torch.float32, device=dev))
+        return *one(f, h), *one(f, h), *one(h, f)
+
+    x = torch.ones((t, h), dtype=torch.bfloat16, device=dev)
+    logits = torch.randn((t, experts), device=dev)
+    gate = torch.ones(t, dtype=torch.bfloat16, device=dev)
+    bank, shared = moe.ExpertWeights(*weights(experts)), moe.SharedExpert(*weights())
+    names = launched(lambda: moe.shared_expert_moe(x, logits, gate, bank, shared, top=4))
+    products = [name for name in names if name.startswith("expert_")]
+    assert len(products) == 2, names
+    assert products[0].startswith(f"expert_{kernel}_kernel<"), names
