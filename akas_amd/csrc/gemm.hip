@@ -1007,7 +1007,13 @@ static float dense_cost(const DenseTileCost& c, const DenseArgs& a, int parts) {
 }
 
 // The tile with the least estimate, and the estimate.  The 256x256 kernel is
-// for prefill (above 256 rows), where it fits.
+// for prefill (above 256 rows), where it fits.  Past one round of it the
+// estimates, which are close to each other there, favour the small tiles too
+// often (M=8192, K=1024, N=8192: 95 us, 128x128 113; M=4100, K=768, N=6144:
+// 32.5, 35.6), so from three k-blocks they only decide where its last round is nearly empty: an
+// eighth of the CUs or less after one round (M=5571, K=2048, N=3072: 59.5,
+// 55.2), or after two at up to eight k-blocks (M=5571, N=6144: K=768 48.1,
+// 45.0, K=1536 76.5, 78.1).
 static DenseTile dense_tile(const DenseArgs& a, int parts, float* cost = nullptr) {
   int best = kTile64x64;
   float least = dense_cost(kDenseTileCost[best], a, parts);
@@ -1018,6 +1024,13 @@ static DenseTile dense_tile(const DenseArgs& a, int parts, float* cost = nullptr
       least = t;
       best = i;
     }
+  }
+  if (best != kTile256x256 && a.M > 256 && a.kb_per_part > 2 && dma_fits(a)) {
+    const int64_t cus = device_cus();
+    const int64_t tiles = (int64_t)((a.M + 255) / 256) * ((a.N + 255) / 256) * parts;
+    const int64_t full = tiles / cus, rest = tiles % cus;
+    const bool tail = rest > 0 && rest * 8 <= cus && (full == 1 || (full == 2 && a.kb_per_part <= 8));
+    if (tiles > cus && !tail) best = kTile256x256;
   }
   if (cost) *cost = least;
   return (DenseTile)best;

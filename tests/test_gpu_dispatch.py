@@ -47,6 +47,23 @@ def test_staged_kernels(dev, launched, m, k, n, offset, kernel):
     assert names and all(name.startswith(kernel) for name in names), names
 
 
+# Prefill tiles past one round of 256x256 ones: those, unless their last round
+# is nearly empty.
+@pytest.mark.parametrize("m,k,n,kernel", [
+    (8192, 1024, 8192, "dense_dma_kernel<"),
+    (4100, 768, 6144, "dense_dma_kernel<"),
+    (7000, 2048, 3072, "dense_dma_kernel<"),
+    (4096, 512, 4096, "dense_dma_kernel<"),  # one full round
+    (4100, 512, 4096, "dense_pipe_kernel<"),  # 16 tiles over
+    (3000, 1024, 6144, "dense_pipe_kernel<"),  # 32 over
+    (5571, 768, 6144, "dense_pipe_kernel<"),  # two rounds and 16
+    (5571, 1536, 6144, "dense_dma_kernel<"),
+])
+def test_prefill_tiles(dev, launched, m, k, n, kernel):
+    names = launched(_linear(dev, m, k, n, quantized=True))
+    assert len(names) == 1 and names[0].startswith(kernel), names
+
+
 def _experts(dev, t, h, f, experts, top, *, offset=0):
     """The gate/up and down products of a routed batch, as calls without
     arguments; codes start ``offset`` bytes off 16-byte alignment."""
