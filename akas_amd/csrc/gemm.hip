@@ -950,8 +950,8 @@ static void launch_tiled(const DenseArgs& a, int parts, hipStream_t s) {
       <<<dim3(tiles, parts), 64 * WMW * WNW, 0, s>>>(a);
 }
 
-// What the DMA-fed 256x256 kernel accepts: whole 128-column blocks and output
-// rows aligned for its 16-byte stores.
+// What the DMA-fed 256x256 kernel accepts beside what pipe_fits asks: whole
+// 128-column blocks and output rows aligned for its 16-byte stores.
 static bool dma_fits(const DenseArgs& a) {
   const int esz = a.out_dtype == AKAS_DTYPE_F32 ? 4 : 2;
   return a.N % 128 == 0 && a.kb_per_part <= dma::MAX_KB && (a.ldo * esz) % 16 == 0 &&
@@ -1012,10 +1012,10 @@ static float dense_cost(const DenseTileCost& c, const DenseArgs& a, int parts) {
 // for prefill (above 256 rows), where it fits.  Past one round of it the
 // estimates, which are close to each other there, favour the small tiles too
 // often (M=8192, K=1024, N=8192: 95 us, 128x128 113; M=4100, K=768, N=6144:
-// 32.5, 35.6), so from three k-blocks they only decide where its last round is nearly empty: an
-// eighth of the CUs or less after one round (M=5571, K=2048, N=3072: 59.5,
-// 55.2), or after two at up to eight k-blocks (M=5571, N=6144: K=768 48.1,
-// 45.0, K=1536 76.5, 78.1).
+// 32.5, 35.6), so from three k-blocks they only decide where its last round is
+// nearly empty: an eighth of the CUs or less after one round (M=5571, K=2048,
+// N=3072: 59.5, 55.2), or after two at up to eight k-blocks (M=5571, N=6144:
+// K=768 48.1, 45.0, K=1536 76.5, 78.1).
 static DenseTile dense_tile(const DenseArgs& a, int parts, float* cost = nullptr) {
   int best = kTile64x64;
   float least = dense_cost(kDenseTileCost[best], a, parts);

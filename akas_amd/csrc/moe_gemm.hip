@@ -1297,19 +1297,28 @@ static void launch_expert_dma(ExpertArgs a, hipStream_t s) {
   expert_dma_kernel<MODE, OUT><<<grid, dma::THREADS, 0, s>>>(a);
 }
 
+// Both DMA engines copy 16 bytes a lane straight to LDS, which takes code rows
+// on 16-byte boundaries (rows are multiples of 128 bytes, so the bases').
+// Other codes go through registers.
+static bool codes_aligned(const ExpertArgs& a) {
+  for (const uint8_t* p : {a.x, a.w, a.w2, a.xw, a.xw2})
+    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
+  return true;
+}
+
 // The DMA-fed 256-row tiles (prefill batches); its 16-byte stores need a
 // 16-byte aligned output.
 static bool expert_dma_fits(const ExpertArgs& a, int64_t n_mult) {
-  return a.N % n_mult == 0 && a.kb_per_part <= dma::MAX_KB &&
+  return a.N % n_mult == 0 && a.kb_per_part <= dma::MAX_KB && codes_aligned(a) &&
          reinterpret_cast<uintptr_t>(a.out) % 16 == 0;
 }
 
-// The pipelined engine's DMA takes 16-byte aligned codes (rows are multiples
-// of 128 bytes).
+// The pipelined engine; its epilogue stores four FP8 codes at a time (other
+// outputs off alignment it stores element by element).
+template <int MODE>
 static bool expert_pipe_fits(const ExpertArgs& a) {
-  const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  return a.kb_per_part <= kExpertPipeMaxKb && aligned(a.x) && aligned(a.w) && aligned(a.w2) &&
-         aligned(a.xw) && aligned(a.xw2);
+  return a.kb_per_part <= kExpertPipeMaxKb && codes_aligned(a) &&
+         (MODE != kSwigluFp8 || reinterpret_cast<uintptr_t>(a.out) % 4 == 0);
 }
 
 // Whether the 256-row tiles of a batch (column_blocks of them per row tile)
@@ -1346,7 +1355,7 @@ static void launch_partial(const ExpertArgs& a, hipStream_t s) {
   const int64_t mean = (int64_t)a.r * a.top / a.E, slots = 3 * (int64_t)device_cus();
   const int64_t tiles64 = (int64_t)a.E * (a.N / 128) * a.parts;
   const bool full = mean > 40 && mean <= 48 && tiles64 <= slots && tiles64 * 9 / 8 > slots;
-  const bool piped = MODE == kPartial && mean >= 32 && !full && expert_pipe_fits(a);
+  const bool piped = MODE == kPartial && mean >= 32 && !full && expert_pipe_fits<MODE>(a);
   const bool late = piped && (OUT == AKAS_DTYPE_F32 || few_tiles(a, mean, a.N / 256 * a.parts));
   if (routed_mean(a) >= (late ? 128 : 112) && expert_dma_fits(a, dma::BN)) {
     launch_expert_dma<MODE, OUT>(a, s);
@@ -1411,7 +1420,7 @@ static void launch_paired(const ExpertArgs& a, hipStream_t s) {
     // on 128 rows, 15.3 on 64).
     const int64_t column_blocks = a.N / 128 * a.parts;
     const bool few = few_tiles(a, mean, column_blocks);
-    const bool piped = MODE == kSwigluFp8 && expert_pipe_fits(a);
+    const bool piped = MODE == kSwigluFp8 && expert_pipe_fits<MODE>(a);
     const bool one_round = ((int64_t)a.r * a.top / 128 + a.E) * column_blocks <= cus;
     const int64_t least = few ? (piped && one_round ? 241 : 128) : MODE == kPairPartial ? 120 : 100;
     if (aligned && routed_mean(a) >= least && expert_dma_fits(a, dma::BN / 2)) {

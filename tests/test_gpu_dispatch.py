@@ -172,3 +172,13 @@ def test_shared_block_row_tiles(dev, launched, t, kernel):
     products = [name for name in names if name.startswith("expert_")]
     assert len(products) == 2, names
     assert products[0].startswith(f"expert_{kernel}_kernel<"), names
+
+
+@pytest.mark.parametrize("offset", [0, 8])
+@pytest.mark.parametrize("mean", [56, 110, 300])
+def test_expert_codes_off_alignment(dev, launched, mean, offset):
+    """Neither DMA engine takes codes off 16-byte alignment."""
+    for call in _experts(dev, mean * 16 // 4, 256, 256, 16, 4, offset=offset):
+        names = launched(call)
+        assert len(names) == 1, names
+        assert names[0].startswith("expert_tiled_kernel<") == (offset != 0), names

@@ -95,3 +95,42 @@ def test_expert_tiles_match_single_experts(dev, sizes, h, f, scale_dtype, packed
         err = (down[torch.float32][mask].double() - want).norm() / want.norm().clamp_min(1e-30)
         assert float(err) <= 1e-4, (e, n)  # the FP8 instruction's own sums
     assert torch.equal(down[torch.float32].to(torch.bfloat16), down[torch.bfloat16])
+
+
+@pytest.mark.parametrize("mean", [16, 40, 105, 300])
+def test_expert_operands_off_alignment(dev, mean):
+    """Codes 8 bytes and FP8 outputs one byte off alignment: the aligned
+    call's results, and no byte outside them."""
+    import torch
+    from akas_amd import ops
+
+    experts, top, h, f = 8, 2, 384, 256
+    r = mean * experts // top
+    g = torch.Generator(device=dev)
+    g.manual_seed(mean)
+    w1, s1 = _bank(torch, g, experts, f, h, torch.float32, dev)
+    w3, s3 = _bank(torch, g, experts, f, h, torch.float32, dev)
+    w2, s2 = _bank(torch, g, experts, h, f, torch.float32, dev)
+    ids = torch.rand((r, experts), generator=g, device=dev).topk(top, -1).indices.to(torch.int32)
+    codes, scales = ops.quantize(torch.randn((r, h), generator=g, device=dev))
+    counts, routes = ops.quantized_routes(ids, torch.ones(r, dtype=torch.int32, device=dev),
+                                          experts=experts)
+
+    def off(t, n=8):
+        moved = torch.empty(t.numel() + n, dtype=t.dtype, device=dev)[n:].view(t.shape)
+        return moved.copy_(t)
+
+    kw = dict(r=r, top=top, product_dtype=torch.bfloat16, activation_dtype=torch.bfloat16)
+    act, acs = ops.fp8_expert_swiglu(codes, scales, w1, s1, w3, s3, counts, routes, **kw)
+    down = ops.expert_partial(act, acs, w2, s2, counts, routes, r=r, top=top, routed_input=True)
+    buf = torch.full((r * top * f + 17,), 99, dtype=torch.uint8, device=dev)
+    for x, a, b in ((off(codes), w1, w3), (codes, off(w1), w3), (codes, w1, off(w3)),
+                    (codes, w1, w3)):
+        buf.fill_(99)
+        out = buf[1:1 + act.numel()].view(act.shape)
+        ops.fp8_expert_swiglu(x, scales, a, s1, b, s3, counts, routes, out=out, **kw)
+        assert torch.equal(out, act)
+        assert int(buf[0]) == 99 and bool((buf[1 + act.numel():] == 99).all())
+    for x, w in ((off(act), w2), (act, off(w2))):
+        assert torch.equal(down, ops.expert_partial(x, acs, w, s2, counts, routes, r=r, top=top,
+                                                    routed_input=True))
