@@ -1069,7 +1069,8 @@ static int split_rows(int m) { return m <= 32 ? 16 : m <= 64 ? 32 : m <= 128 ? 6
 // two of its workgroups come to a CU (fp8_linear, K=2048, N=8192: M=64
 // 9.4 us, 11 pipelined; M=128 11.0, 11.4).  Beyond, its time is 4.2 us and its
 // operand bytes per CU at 70 KB per us (measured from 300 to 900 KB per CU):
-// N=8192, M=256 15.9 us, 13.5 pipelined; K=8192, N=6144, M=100 31.5, 27.1.
+// N=8192, M=256 15.9 us, 13.5 pipelined; K=8192, N=6144, M=100 31.5, 27.1;
+// near the line, K=18432, N=2048, M=100 27.1, 29.1.
 static bool split_applies(const DenseArgs& a, int parts) {
   if (a.M <= 16 || a.M > 256 || !split_fits(a) || parts < 1) return false;
   const int nt = split_nt(a), rows = split_rows(a.M), row_tiles = (a.M + rows - 1) / rows;
@@ -1079,7 +1080,7 @@ static bool split_applies(const DenseArgs& a, int parts) {
   const float bytes = (float)blocks * (row_tiles * 16 * nt + a.M) * (a.kb_per_part * kBlock);
   float cost;
   dense_tile(a, parts, &cost);
-  return 4.2f + bytes / 1024.f / device_cus() / 70.f <= 1.1f * cost;
+  return 4.2f + bytes / 1024.f / device_cus() / 70.f <= 1.13f * cost;
 }
 
 template <int MT, int PF, int AFIRST, int AF, int OUT, int SDT, int MH = 1, int NT = kSplitNt>
