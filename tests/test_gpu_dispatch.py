@@ -58,10 +58,53 @@ def test_staged_kernels(dev, launched, m, k, n, offset, kernel):
     (3000, 1024, 6144, "dense_pipe_kernel<"),  # 32 over
     (5571, 768, 6144, "dense_pipe_kernel<"),  # two rounds and 16
     (5571, 1536, 6144, "dense_dma_kernel<"),
+    # below a round, ragged
+    (2000, 512, 7808, "dense_dma_kernel<"), (1537, 384, 9088, "dense_dma_kernel<"),
+    (4097, 256, 3840, "dense_dma_kernel<"), (2304, 1024, 6784, "dense_dma_kernel<"),
 ])
 def test_prefill_tiles(dev, launched, m, k, n, kernel):
     names = launched(_linear(dev, m, k, n, quantized=True))
     assert len(names) == 1 and names[0].startswith(kernel), names
+
+
+# Between decode and prefill: the tiles of the pipelined engine, and what comes
+# before it.
+@pytest.mark.parametrize("m,k,n,kernel", [
+    (17, 128, 512, "dense_small_kernel<2,"),
+    (33, 256, 528, "dense_small_kernel<4,"),
+    (17, 1152, 4128, "dense_wide_kernel<2,"),
+    (32, 1920, 6144, "dense_wide_kernel<2,"),
+    (65, 128, 512, "dense_pipe_kernel<pipe::Engine<64, 64,"),
+    (127, 384, 1040, "dense_pipe_kernel<pipe::Engine<64, 64,"),
+    (300, 2048, 6144, "dense_pipe_kernel<pipe::Engine<64, 128,"),
+    (513, 1408, 6000, "dense_pipe_kernel<pipe::Engine<128, 128, 2, 2, 2,"),
+    (1290, 2048, 2000, "dense_pipe_kernel<pipe::Engine<128, 128, 2, 2, 2,"),
+    (1100, 768, 5008, "dense_pipe_kernel<pipe::Engine<128, 128, 2, 2, 1,"),
+])
+def test_mid_size_tiles(dev, launched, m, k, n, kernel):
+    names = launched(_linear(dev, m, k, n, quantized=True))
+    assert len(names) == 1 and names[0].startswith(kernel), names
+
+
+# fp8_linear past 2048 deep: 2048-deep partitions on the split kernel or the
+# pipelined engine, then the merge; up to 16 rows the fused kernel, or the
+# quantizer and the product.
+@pytest.mark.parametrize("m,k,n,kernels", [
+    (64, 8192, 2048, ("quantize", "dense_split", "merge")),
+    (100, 18432, 2048, ("quantize", "dense_split", "merge")),
+    (200, 8192, 2048, ("quantize", "dense_pipe", "merge")),
+    (64, 8192, 4096, ("quantize", "dense_pipe", "merge")),
+    (256, 4096, 8192, ("quantize", "dense_pipe", "merge")),
+    (1, 8192, 2048, ("dense_wide",)),
+    (8, 2688, 2048, ("dense_wide",)),
+    (16, 2560, 6144, ("dense_wide",)),
+    (8, 8192, 2048, ("quantize", "dense_wide")),
+    (16, 4096, 6144, ("quantize", "dense_wide")),
+])
+def test_deep_linear_kernels(dev, launched, m, k, n, kernels):
+    names = launched(_linear(dev, m, k, n))
+    assert len(names) == len(kernels), names
+    assert all(name.startswith(kernel + "_kernel") for name, kernel in zip(names, kernels)), names
 
 
 def _experts(dev, t, h, f, experts, top, *, offset=0):

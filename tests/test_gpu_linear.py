@@ -148,10 +148,13 @@ def test_fp8_linear_narrow_tiles_match_two_step(dev, m, n):
     assert rel_fro(y.cpu().numpy(), ofp8.fp8_linear(x, codes, scales)) < 1e-4
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 8192, 2048), (8, 8192, 2048), (16, 4096, 6144)])
+@pytest.mark.parametrize("m,k,n", [(1, 8192, 2048), (8, 8192, 2048), (16, 4096, 6144),
+                                   (8, 2688, 2048), (16, 2560, 6144)])
 def test_fp8_linear_deep_k_fused_small(dev, m, k, n):
-    """Up to 16 rows the wide kernel quantizes the whole activation slab into
-    LDS, deep K included (K=8192: a 132 KB slab), within the oracle bound."""
+    """Up to 16 rows the wide kernel holds the whole activation slab in LDS,
+    deep K included (K=8192: a 132 KB slab), within the oracle bound: it
+    quantizes the slab itself, or, of many rows and k-blocks (the second and
+    third shape), takes the quantizer's codes."""
     import torch
     from akas_amd import ops
 
@@ -165,7 +168,9 @@ def test_fp8_linear_deep_k_fused_small(dev, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [(64, 8192, 2048), (17, 4096, 512), (40, 4096, 1040),
-                                   (256, 4096, 6144), (100, 6144, 480), (128, 8192, 2048)])
+                                   (256, 4096, 6144), (100, 6144, 480), (128, 8192, 2048),
+                                   # the partitions on the pipelined engine
+                                   (200, 8192, 2048), (64, 8192, 4096), (256, 4096, 8192)])
 def test_fp8_linear_deep_k_partitions(dev, m, k, n):
     """Deeper than 2048 at 17-256 rows: fp8_linear runs 2048-deep partitions
     with f32 partials and the serial merge -- bit for bit the
@@ -233,10 +238,12 @@ def test_fp8_linear_config1_and_out_dtypes(dev, out_dtype):
     assert rel_fro(got, exp) < (1e-4 if out_dtype == "float32" else 4e-3)
 
 
-# Shapes that select the DMA-fed 256x256 prefill kernel (more than 256 rows,
-# N a multiple of 128, at least 240 tiles): ragged last row tiles (M % 256 of
-# 1, 16 and 208 rows) and a half-width last column tile (N % 256 == 128).
-DMA_CASES = [(2000, 512, 7808), (1537, 384, 10112), (4097, 256, 3840), (2304, 1024, 6784)]
+# Shapes of the DMA-fed 256x256 prefill kernel (more than 256 rows, N a multiple
+# of 128, just under a round of its tiles): ragged last row tiles (M % 256 of 1
+# and 208 rows) and a half-width last column tile (N % 256 == 128).  The second
+# leaves its last round nearly empty and runs on 128x128 pipelined tiles.
+DMA_CASES = [(2000, 512, 7808), (1537, 384, 10112), (4097, 256, 3840), (2304, 1024, 6784),
+             (1537, 384, 9088)]
 
 
 @pytest.mark.parametrize("m,k,n", DMA_CASES)

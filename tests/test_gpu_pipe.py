@@ -37,9 +37,11 @@ def _problem(dev, m, k, n, seed, scale_dtype="float32"):
 
 
 @pytest.mark.parametrize("m,k,n", [
+    # few rows and k-blocks: the direct small kernel
+    (17, 128, 512), (33, 256, 528), (63, 384, 1040),
     # 64x64 tiles in two k-block groups: one row past a tile, one short of
     # it, ragged columns, 1 to 5 and 17 k-blocks (four stages of two)
-    (17, 128, 512), (33, 256, 528), (63, 384, 1040), (65, 512, 2000), (127, 640, 2048),
+    (65, 128, 512), (65, 256, 528), (127, 384, 1040), (65, 512, 2000), (127, 640, 2048),
     (257, 2176, 80), (300, 1152, 1008),
     # 64x128 tiles (three stages of two)
     (300, 2048, 6144), (641, 1280, 2064), (999, 896, 2048), (770, 384, 1936),
@@ -111,3 +113,29 @@ def test_mid_size_unaligned_operands(dev, m, n, out_dtype):
     shifted.copy_(codes)
     got = ops.fp8_linear(shifted, wc, ws, activation_scales=scales, out_dtype=dt)
     assert _rel(got.float().cpu().numpy(), want) <= tol
+
+
+@pytest.mark.parametrize("m,k,n", [(17, 1152, 4128), (24, 1536, 6144), (25, 1920, 4128),
+                                   (32, 1152, 6144)])
+@pytest.mark.parametrize("scale_dtype", ["float32", "bfloat16"])
+def test_wide_rows_exact_products(dev, m, k, n, scale_dtype):
+    """17 to 32 rows of 9 to 15 k-blocks on the wide kernel, codes on and off
+    16-byte alignment: exact products with binary scales, so the output equals
+    the float64 oracle bit for bit."""
+    import torch
+    from akas_amd import ops
+    from golden_inputs import exact_codes
+
+    rng = np.random.default_rng(m + k + n)
+    x, w = exact_codes(rng, (m, k)), exact_codes(rng, (n, k))
+    xs = (2.0 ** rng.integers(-4, 2, (m, k // 128))).astype(np.float32)
+    ws = (2.0 ** rng.integers(-4, 2, ((n + 127) // 128, k // 128))).astype(np.float32)
+    want = ofp8.fp8_linear(x, w, ws, activation_scales=xs)
+    wt, xst = torch.from_numpy(w).to(dev), torch.from_numpy(xs).to(dev)
+    wst = torch.from_numpy(ws).to(dev).to(getattr(torch, scale_dtype))
+    for offset in (0, 8):
+        raw = torch.empty(m * k + offset, dtype=torch.uint8, device=dev)
+        xt = raw[offset:].view(m, k)
+        xt.copy_(torch.from_numpy(x))
+        got = ops.fp8_linear(xt, wt, wst, activation_scales=xst)
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
