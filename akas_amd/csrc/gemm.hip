@@ -1255,9 +1255,9 @@ static void launch_staged(const DenseArgs& a, int parts, hipStream_t s) {
 //   16 < M <= 256 with 2048-deep partitions   the split kernel, where estimated
 //                                             faster than the engine below
 //   16 < M <= 64, few k-blocks                the direct small kernel (shallow_rows)
-//   16 < M <= 32, 9 to 16 k-blocks            the wide kernel (K=1536, N=6144,
-//                                             M=24: 6.6 us, 7.0 pipelined;
-//                                             K=1920, N=1536, M=20: 6.2, 7.0)
+//   16 < M <= 32, 9 k-blocks or more,         the wide kernel (M=24: K=1536,
+//     while its slab fits (38)                N=6144 6.6 us, 7.0 pipelined;
+//                                             K=4608, N=3072 11.8, 14.3)
 //   otherwise                                 the pipelined engine or the 256x256
 //                                             DMA kernel, the tile estimated fastest
 // Codes off 16-byte alignment and partitions past kPipeMaxKb k-blocks take
@@ -1273,7 +1273,7 @@ static void launch_dense_t(const DenseArgs& a, int parts, hipStream_t s) {
     launch_staged<OUT, SDT>(a, parts, s);
     return;
   }
-  if (a.M <= 32 && a.kb_per_part > 8 && a.kb_per_part <= 16 && !shallow_rows(a) &&
+  if (a.M <= 32 && a.kb_per_part > 8 && !shallow_rows(a) &&
       launch_wide<2, 2, 8, OUT, SDT>(a, parts, s))
     return;
   if (a.M <= 16 || shallow_rows(a)) {

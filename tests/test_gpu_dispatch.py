@@ -76,6 +76,8 @@ def test_prefill_tiles(dev, launched, m, k, n, kernel):
     (32, 1920, 6144, "dense_wide_kernel<2,"),
     (20, 1920, 1536, "dense_wide_kernel<2,"),
     (20, 1536, 1536, "dense_small_kernel<2,"),
+    (32, 4864, 3072, "dense_wide_kernel<2,"),
+    (32, 4992, 3072, "dense_pipe_kernel<"),  # past its slab
     (65, 128, 512, "dense_pipe_kernel<pipe::Engine<64, 64,"),
     (127, 384, 1040, "dense_pipe_kernel<pipe::Engine<64, 64,"),
     (300, 2048, 6144, "dense_pipe_kernel<pipe::Engine<64, 128,"),

@@ -116,10 +116,10 @@ def test_mid_size_unaligned_operands(dev, m, n, out_dtype):
 
 
 @pytest.mark.parametrize("m,k,n", [(17, 1152, 4128), (24, 1536, 6144), (25, 1920, 4128),
-                                   (32, 1152, 6144)])
+                                   (32, 1152, 6144), (20, 1920, 544), (32, 4864, 96)])
 @pytest.mark.parametrize("scale_dtype", ["float32", "bfloat16"])
 def test_wide_rows_exact_products(dev, m, k, n, scale_dtype):
-    """17 to 32 rows of 9 to 15 k-blocks on the wide kernel, codes on and off
+    """17 to 32 rows of 9 to 38 k-blocks on the wide kernel, codes on and off
     16-byte alignment: exact products with binary scales, so the output equals
     the float64 oracle bit for bit."""
     import torch
