@@ -760,8 +760,9 @@ __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) 
   // So lane l loads that of the wave's l-th k-block once, ahead of the
   // weights, and each use converts its own (fp8_linear, eight slots, M=1, us:
   // K=N=4096 8.0 -> 6.4; K=4096, N=12288 18.7 -> 14.5; two slots 7.0, 15.6).
-  // At most 77 k-blocks fit the slab, ten per wave.
-  constexpr bool LANE_SCALES = SDT == AKAS_DTYPE_BF16 && CW % 16 == 0;
+  // At most 77 k-blocks fit the slab, ten per wave.  Two slots keep a load
+  // each, raw, too (K=2048, N=8192, M=8 6.6 us, 6.8 by lane).
+  constexpr bool LANE_SCALES = SDT == AKAS_DTYPE_BF16 && CW % 16 == 0 && B > 2;
   uint32_t wlane = 0;
   if constexpr (LANE_SCALES) {
     wlane = reinterpret_cast<const uint16_t*>(p.ws)[ws_base + kb0 + min(ks + KS * lane, kbp - 1)];
