@@ -815,10 +815,10 @@ __global__ __launch_bounds__(64 * NTW * KS) void dense_wide_kernel(DenseArgs p) 
       const int halves = (p.M + 7) / 8;
       for (int c = wave; c < kbp * halves; c += NTW * KS) {
         const int lk = c / halves, r0 = (c % halves) * 8, row = r0 + (lane >> 3);
-        const int ch = (lane & 7) ^ pipe::swizzle(row);
+        const int ch = (lane & 7) ^ swizzle(row);
         __builtin_amdgcn_global_load_lds(
             (const void*)(p.a + (int64_t)min(row, p.M - 1) * p.K + (int64_t)(kb0 + lk) * kBlock + ch * 16),
-            (pipe::lds_void*)(lds_a + (size_t)lk * ROWS * 128 + r0 * 128), 16, 0, 0);
+            (lds_void*)(lds_a + (size_t)lk * ROWS * 128 + r0 * 128), 16, 0, 0);
       }
     } else {
       for (int c = tid; c < p.M * kbp * 8; c += THREADS) {

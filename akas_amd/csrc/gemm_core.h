@@ -24,7 +24,11 @@
 
 namespace akas {
 
-AKAS_DEV int lds_off(int row, int chunk) { return row * 128 + ((chunk ^ ((row & 7) ^ ((row >> 3) & 1))) << 4); }
+// What the DMA builtins take as their LDS destination.
+typedef __attribute__((address_space(3))) void lds_void;
+
+AKAS_DEV int swizzle(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+AKAS_DEV int lds_off(int row, int chunk) { return row * 128 + ((chunk ^ swizzle(row)) << 4); }
 
 // Staging plan: every thread moves CA chunks of the A tile and CB chunks of
 // the B tile per k-block.  Thread t owns chunk column (t % 8) of rows

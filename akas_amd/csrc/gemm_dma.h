@@ -30,15 +30,13 @@
 // and the epilogue writes 4 adjacent columns per lane.
 #pragma once
 
-#include "common.h"
+#include "gemm_core.h"
 
 namespace akas {
 namespace dma {
 
 constexpr int BM = 256, BN = 256, THREADS = 512;
 constexpr int STAGE = (BM + BN) * 128;
-
-typedef __attribute__((address_space(3))) void lds_void;
 
 static __shared__ __attribute__((aligned(1024))) uint8_t stage0[STAGE];
 static __shared__ __attribute__((aligned(1024))) uint8_t stage1[STAGE];
@@ -52,13 +50,10 @@ static __shared__ __attribute__((aligned(16))) float wtab[2][MAX_KB];
 template <int S> AKAS_DEV uint8_t* stage_base() { return S ? stage1 : stage0; }
 template <int S> AKAS_DEV float* stage_scales() { return S ? scales1 : scales0; }
 
-AKAS_DEV int swizzle(int row) { return (row & 7) ^ ((row >> 3) & 1); }
-AKAS_DEV int tile_off(int row, int chunk) { return row * 128 + ((chunk ^ swizzle(row)) << 4); }
-
 AKAS_DEV v8i fragment(const uint8_t* tile, int row0, int lane) {
   const int row = row0 + (lane & 15), g = lane >> 4;
-  const u32x4 lo = *reinterpret_cast<const u32x4*>(tile + tile_off(row, 2 * g));
-  const u32x4 hi = *reinterpret_cast<const u32x4*>(tile + tile_off(row, 2 * g + 1));
+  const u32x4 lo = *reinterpret_cast<const u32x4*>(tile + lds_off(row, 2 * g));
+  const u32x4 hi = *reinterpret_cast<const u32x4*>(tile + lds_off(row, 2 * g + 1));
   v8i f;
   f[0] = lo[0]; f[1] = lo[1]; f[2] = lo[2]; f[3] = lo[3];
   f[4] = hi[0]; f[5] = hi[1]; f[6] = hi[2]; f[7] = hi[3];

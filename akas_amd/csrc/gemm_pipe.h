@@ -16,10 +16,15 @@
 //   * G groups of waves take G k-blocks of the same tile per step, so a step
 //     moves G times the bytes per barrier and a tile's k-loop is G times
 //     shorter; their partial tiles are summed in group order in the epilogue.
-// Steady state is then the CU's L2-to-LDS rate: 57-66 GB/s per CU in every
-// configuration measured here (the outstanding-miss limit of its L1), so
-// what is left is choosing the tile that covers the CUs with the fewest bytes
-// (dense_cost in gemm.hip).
+// Steady state is then the rate at which the copies land: 57-66 GB/s per CU
+// in every configuration measured here, about half of what line-wide loads
+// into registers reach in the split kernel (gemm.hip).  The L1s have misses
+// pending for 14 to 17% of the cycles only, and four fifths of the requests
+// hit in L2; what holds it has not been found.  What is left is choosing the tile that covers the CUs with the
+// fewest bytes (dense_cost in gemm.hip).  The weight scales that the dense
+// kernel holds in registers are first used in the k-loop, where the compiler
+// waits for every load before it: the stages ahead of the first step land
+// together.
 //
 // The same launch, 128x128 register-staged tiles -> this engine
 // (GEMM alone, us): M=300 K=2048 N=6144 20.3 -> 10.9; M=512 K=2048 N=2048
@@ -41,10 +46,6 @@
 
 namespace akas {
 namespace pipe {
-
-typedef __attribute__((address_space(3))) void lds_void;
-
-AKAS_DEV int swizzle(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
 // Waits until at most N of the wave's global loads and none of its LDS
 // accesses are outstanding (s_waitcnt: vmcnt N, lgkmcnt 0).

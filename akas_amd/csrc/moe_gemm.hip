@@ -974,8 +974,9 @@ __global__ __launch_bounds__(dma::THREADS) void expert_dma_kernel(ExpertArgs p) 
 }
 
 // ---------------------------------------------------------------------------
-// Experts of about fifty to a hundred rows each, on the pipelined engine
-// (gemm_pipe.h) with one k-block group, so every (row, column) is still one
+// Experts of 32 to 111 mean rows (down) or 49 to 99 (gate/up), and to 127 or
+// 240 where larger tiles would be few (launch_partial, launch_paired), on the
+// pipelined engine (gemm_pipe.h) with one k-block group, so every (row, column) is still one
 // f32 chain in ascending k-block order and the results are those of the other
 // grouped kernels bit for bit.  Modes kPartial and kSwigluFp8.
 //
@@ -984,9 +985,12 @@ __global__ __launch_bounds__(dma::THREADS) void expert_dma_kernel(ExpertArgs p) 
 // in flight.  64 experts x 1536 x 2048, bf16 intermediates, GEMMs alone in
 // us: gate/up 111.8 -> 95.7 at 900 tokens x 4, 112.1 -> 104.3 at 1500; down
 // 45.3 -> 41.1, 47.7 -> 44.9.  The first stages' weights are requested before
-// the tile's rows are known.  (Chaining a workgroup's items, the next one's
-// weights requested under the epilogue, measured 98.7 / 107.6: the load rate
-// inside the k-loop, not the gaps between tiles, is what holds them.)
+// the tile's rows are known; the routes' first use then waits for those
+// weights too (the loads stand behind branches on the routing form, so the
+// compiler waits for all), and the rows' copies follow.  (Chaining a
+// workgroup's items, the next one's weights requested under the epilogue,
+// measured 98.7 / 107.6: the load rate inside the k-loop, not the gaps between
+// tiles, is what holds them.)
 // ---------------------------------------------------------------------------
 constexpr int kExpertPipeMaxKb = 128;
 

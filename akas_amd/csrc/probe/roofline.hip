@@ -6,7 +6,8 @@
 //                  stored only if it matches a sentinel (so the loads stay but
 //                  nothing is written);
 //   mfma        -- back-to-back FP8 MFMAs (16x16x128, OCP e4m3 operands in
-//                  registers) on four independent accumulators per wave;
+//                  registers, the form without block scales that the path
+//                  issues) on four independent accumulators per wave;
 //   load_mix    -- the loads of the decode split GEMM (16 < M <= 256,
 //                  K = 2048) without its products, its LDS staging or its
 //                  stores: the same workgroups, waves, tile order, load
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(kThreads) void mfma_kernel(uint32_t* __restrict__ s
   for (int it = 0; it < iters; ++it) {
 #pragma unroll
     for (int c = 0; c < kChains; ++c)
-      acc[c] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc[c], 0, 0, 0, 127, 0, 127);
+      acc[c] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc[c], 0, 0, 0, 0, 0, 0);
   }
   float s = 0.f;
 #pragma unroll
